@@ -330,3 +330,49 @@ def run(state):
     else:
         out = ops.paged_attention_prefill(q, s["k_cache"], s["v_cache"], s["table"], s["lens"], s["cum"], s["alibi"], s["scale"])
     return (out, *written)
+
+
+# ---- the same in 64 bits ----
+
+def _rotated(x, pos, sin, cos):
+    """GPT-NeoX rotation of x [tokens, heads, head] in 64 bits."""
+    half = x.shape[-1] // 2
+    sin, cos = sin[pos].double()[:, None, :], cos[pos].double()[:, None, :]
+    lo, hi = x[..., :half].double(), x[..., half:].double()
+    return torch.cat((lo * cos - hi * sin, lo * sin + hi * cos), dim=-1)
+
+
+def exact(case, seed):
+    if case["op"] == "write":
+        return None  # moved bytes, and a rotation whose roundings are prescribed: compared bit by bit
+    s = prepare(case, seed)
+    q, k_cache, v_cache = s["q"], s["k_cache"], s["v_cache"]
+    more = ()
+    if case["op"].endswith("_step"):
+        # the rotated vectors go through the storage type: that is what the caches and the rotated query hold
+        q_rot = _rotated(q, s["pos"], s["sin"], s["cos"])
+        k_rot = _rotated(s["k"], s["pos"], s["sin"], s["cos"]).to(k_cache.dtype)
+        page, row = s["slots"] // case["page"], s["slots"] % case["page"]
+        k_cache[page, :, row], v_cache[page, :, row] = k_rot, s["v"]
+        q = q_rot.to(q.dtype)
+        more = (None, None, q_rot)
+    new, _ = _lengths(case)
+    lens = s["lens"].tolist()
+    cum = s["cum"].tolist() if "cum" in s else list(range(len(new) + 1))
+    kv, group = case["kv_heads"], case["heads"] // case["kv_heads"]
+    out = torch.empty((*q.shape[:-1], case["value"]), dtype=torch.float64, device=q.device)
+    for i, total in enumerate(lens):
+        pages = s["table"][i, :-(-total // case["page"])].long()
+        n = cum[i + 1] - cum[i]
+        last = torch.arange(total - n, total, device=q.device)  # the last token that each new token sees
+        away = torch.arange(total, device=q.device)[None, :] - last[:, None]
+        for g in range(kv):
+            k = k_cache[pages, g].reshape(-1, case["head"])[:total].double()
+            v = v_cache[pages, g].reshape(-1, case["value"])[:total].double()
+            for h in range(g * group, (g + 1) * group):
+                scores = (q[cum[i]:cum[i + 1], h].double() @ k.T) * s["scale"]
+                if s["alibi"] is not None:
+                    scores = scores + s["alibi"][h].double() * away
+                scores.masked_fill_(away > 0, -math.inf)
+                out[cum[i]:cum[i + 1], h] = torch.softmax(scores, dim=-1) @ v
+    return (out, *more)
