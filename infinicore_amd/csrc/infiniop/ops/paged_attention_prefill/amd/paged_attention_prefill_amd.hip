@@ -8,6 +8,7 @@
 #include "../../../devices/amd/amd_device.h"
 #include "prefill_common.h"
 #include "prefill_generic.h"
+#include "prefill_latent.h"
 #include "prefill_tiled.h"
 #include <cstdlib>
 #include <cstring>
@@ -68,15 +69,27 @@ Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo
     if (rows_per_seq <= 64 || rows / 128 * static_cast<long long>(in.num_kv_heads) < resident * dev.compute_units) {
         r = 1;
     }
+    if (latent) {
+        // Latent attention: one workgroup per compute unit with either kernel, and a round of 128-row workgroups
+        // (prefill_latent.h) takes 1.4 x as long as a round of 64-row ones (kv 2 200, 16 heads: 164 us against 119 us).
+        // So 128 rows where they save more than a third of the rounds. Measured, 64 rows against 128, by 64-row blocks:
+        // 256 (one round either way) 119 / 164 us, 300 202 / 166, 512 228 / 189, 520 (3 rounds / 2) 290 / 299,
+        // 770 407 / 343, 1 100 571 / 480; 400 sequences of 8 new tokens 342 / 244.
+        const long long units = dev.compute_units > 0 ? dev.compute_units : 1;
+        const long long streams = seqs * static_cast<long long>(in.num_kv_heads);
+        const long long rounds64 = (streams * ((rows_per_seq + 63) / 64) + units - 1) / units;
+        const long long rounds128 = (streams * ((rows_per_seq + 127) / 128) + units - 1) / units;
+        r = 2 * rounds64 > 3 * rounds128 ? 2 : 1;
+    }
     if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_GROUPS")) {
         const int forced = std::atoi(env);
         if (forced == 1 || forced == 2) {
             r = forced;
         }
     }
-    if (latent) {
-        // the accumulators of 64 rows x 512 (576) columns are half the register file: there is no kernel with two
-        // groups, whatever the knob says (grid and kernel must agree on the rows per workgroup)
+    if (latent && (in.value_size != 512 || in.has_alibi || !(in.scale > 0.0f))) {
+        // 128 rows have a kernel of their own (prefill_latent.h) for values of 512 without ALiBi only, whatever the
+        // knob says (grid and kernel must agree on the rows per workgroup)
         r = 1;
     }
     plan.groups_per_wave = r;
@@ -101,12 +114,19 @@ template <typename T, typename Tindex, int KHEAD, int VHEAD, bool PLAIN>
 void launchTiledHead(const PrefillArgs &a, const Plan &plan, hipStream_t stream) {
     // sum over sequences of ceil(rows / block_rows) is at most floor(total rows / block_rows) + num_seqs
     const long long rows = static_cast<long long>(a.total_q_tokens) * a.group;
-    const int groups = plan.groups_per_wave;
+    const int groups = KHEAD == 576 && !PLAIN ? 1 : plan.groups_per_wave; // slopes handed over unannounced
     const int block_rows = prefillBlockRows(groups);
+    static_assert(prefillBlockRows(2) == kLatentRows);
     const dim3 grid(static_cast<unsigned>((rows / block_rows + a.num_seqs) * a.num_kv_heads));
     if constexpr (KHEAD == VHEAD && KHEAD <= 256) {
         if (groups == 2) {
             prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 2, PLAIN><<<grid, kPrefillThreads, 0, stream>>>(a);
+            return;
+        }
+    }
+    if constexpr (KHEAD == 576 && VHEAD == 512 && PLAIN) {
+        if (groups == 2) {
+            prefillLatentKernel<T, Tindex><<<grid, kLatentThreads, 0, stream>>>(a);
             return;
         }
     }

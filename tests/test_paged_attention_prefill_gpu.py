@@ -176,6 +176,35 @@ def test_mla_column_layout_and_garbage(gpu_handle, oracle):
     assert torch.allclose(got, want, atol=2e-3 * float(ramp.float().abs().max()), rtol=0), (got - want).abs().max()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,Hkv,bs,new,history", [
+    (16, 1, 16, (1, 8), (0, 31)),       # less than one block of 128 rows, one to three steps of 32 tokens
+    (16, 1, 16, (8, 9), (23, 24)),      # exactly 128 rows and 144; kv lengths 31..33: one step, one token into the next
+    (5, 1, 8, (1, 150), (0, 300)),      # pages of 8: two per tile; rows of a token split over row blocks
+    (20, 2, 32, (1, 150), (0, 300)),
+    (16, 1, 64, (60, 200), (1000, 2300)),  # more than 64 table entries of 16 tokens, many steps
+])
+def test_mla_128_rows_per_workgroup(gpu_handle, oracle, monkeypatch, H, Hkv, bs, new, history, dtype):
+    """The eight-wavefront kernel of the latent shape on scores that climb (every wavefront rescales in its own steps),
+    garbage behind the sequences, and the ALiBi call that has no such kernel."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", "2")
+    inp = workloads.make_prefill_inputs(prefill_config(f"mla128_{H}_{bs}", dtype, 3, H, Hkv, 576, bs, new, history, seed=570 + bs))
+    inp.v_cache = inp.v_cache[..., :512].contiguous()
+    for s in range(3):
+        L = int(inp.seq_lens[s])
+        if L % bs:
+            page = int(inp.block_tables[s, (L - 1) // bs])
+            inp.k_cache[page, :, L % bs:, :] = float("nan")
+            inp.v_cache[page, :, L % bs:, :] = float("nan")
+        for j in range(0, L, bs):
+            inp.k_cache[int(inp.block_tables[s, j // bs])] *= 0.25 + 3.0 * j / L
+    rows = sample_rows(inp) if history[1] > 1000 else None
+    run_case(gpu_handle, oracle, inp, rows=rows)
+    if bs == 8:
+        slopes = torch.tensor([2.0 ** (-(h + 1) / 2) for h in range(H)], dtype=torch.float32)
+        run_case(gpu_handle, oracle, inp, alibi=slopes, index_dtype=torch.int32)
+
+
 # ---- heads of 576 with values of 576 (the decode test list of the reference has the shape,
 # test/infiniop/paged_attention.py:106): the matrix-core kernel of the latent shape with 36 value blocks -------------
 
