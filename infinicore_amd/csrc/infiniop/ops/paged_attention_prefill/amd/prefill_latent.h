@@ -14,9 +14,10 @@
 //     register layout they are computed and used in, the rescaling factors of a step beside them.
 // Per step of 32 tokens and 128 rows: 288 KiB of K, 64 KiB of V and 32 KiB of probabilities out of LDS (3 072 clocks),
 // 2 208 clocks of matrix instructions per SIMD. 128 accumulator and 72 query registers per lane leave room for two
-// wavefronts per SIMD; the compiler still keeps one query operand and a few addresses in scratch memory.
-// Measured (16 sequences, 16 heads, 128 - 512 new tokens over 1 024 - 8 192 of history, bf16): 1 378 -> 1 034 us
-// (594 -> 792 TFLOP/s); with K in one run of 72 chunks per row, whose reads meet in the banks two at a time, 1 270 us.
+// wavefronts per SIMD, and 56 for everything else: nothing of the loop is in scratch memory (a reload there waits for the
+// direct loads in flight too: with one query operand reloaded behind them the case below took 1 287 us).
+// Measured (16 sequences, 16 heads, 128 - 512 new tokens over 1 024 - 8 192 of history, bf16; the kernels in turn on
+// one GPU): 1 391 -> 1 006 us (589 -> 814 TFLOP/s); with K in one run of 72 chunks per row, whose reads meet in the banks two at a time, 1 270 us.
 // By the counts above LDS is the longest of the pipes: the K operands, read once per 16 rows, are three quarters of it.
 // Everything else (block search, page ids, LDS layouts, masks, lazy reference point) is as in
 // prefill_tiled.h.
@@ -200,7 +201,9 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
             if (t + row < kv_len) {
                 loadLane16ToLds(src, v_dst + 64 * i);
             } else {
-                v_dst[64 * i + own] = make_uint4(0, 0, 0, 0);
+                uint32_t zero = 0;
+                asm volatile("" : "+v"(zero)); // not four registers of zeros for the whole loop
+                v_dst[64 * i + own] = make_uint4(zero, zero, zero, zero);
             }
         }
     };
@@ -232,8 +235,6 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
                            + 256 * kCols * quarter;
     // slots of chunk g of row c in either part of a K tile; chunk 4 kk + g is 4 (kk % 4) XORed and 16 (kk / 4) added
     const int k_first = 64 * c + (g ^ c), k_last = 64 * 16 + 8 * c + (g ^ (c >> 1));
-    const uint32_t one2 = T::pack2(1.0f, 1.0f);
-    const uint4 ones = make_uint4(one2, one2, one2, one2);
     const float unit = a.scale_log2;
     const float lazy = kLazyLog2 / unit;
 
@@ -242,15 +243,19 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
         {
             constexpr int kAheadK = 3; // two wavefronts of the SIMD take turns; a fourth would be spilled
             constexpr int kOperandsK = 2 * G::kLoadsK;
-            // operand idx: 32 dimensions kkOf(idx) of tile idx % 2 (neighbours go to different accumulators). The
-            // dimensions that share a lane address follow one another: one address is live, not four.
-            auto kkOf = [](int idx) { return idx / 2 < 16 ? 4 * (idx / 2 % 4) + idx / 8 : idx / 2; };
-            int first = k_first;
+            // operand idx: the 32 dimensions kk = idx / 2 of tile idx % 2 (neighbours go to different accumulators), added in
+            // the order of prefillTiledKernel, so that the outputs of the two are the same bits. Four lane addresses would
+            // serve the sixteen dimensions of the first part of a row: each is formed from the one before, one is live.
+            int first = 16 * k_first;
             asm volatile("" : "+v"(first));
             auto readK = [&](int idx) {
-                const int kk = kkOf(idx);
-                const int slot = kk < 16 ? (first ^ (4 * (kk % 4))) + 16 * (kk / 4) : k_last ^ (4 * (kk % 4));
-                return lds.k[buf][idx % 2 * kTileChunksK + slot];
+                const int kk = idx / 2;
+                if (idx % 2 == 0 && kk > 0 && kk < 16) {
+                    first ^= 16 * (4 * (kk % 4) ^ 4 * ((kk - 1) % 4));
+                    asm volatile("" : "+v"(first));
+                }
+                const int at = kk < 16 ? first + 16 * 16 * (kk / 4) : 16 * (k_last ^ (4 * (kk % 4)));
+                return *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(lds.k[buf] + idx % 2 * kTileChunksK) + at);
             };
             uint4 kf[kAheadK];
 #pragma unroll
@@ -265,7 +270,7 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
                     kf[idx % kAheadK] = readK(idx + kAheadK);
                     __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 }
-                s[idx % 2] = T::mfmaK32(cur, q_reg[kkOf(idx)], s[idx % 2]);
+                s[idx % 2] = T::mfmaK32(cur, q_reg[idx / 2], s[idx % 2]);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 if (idx % 4 == 3) {
                     issueSlot(idx / 4);
@@ -315,7 +320,9 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
         }
         const uint4 p_own = make_uint4(wds[0], wds[1], wds[2], wds[3]);
         lds.p[w][lane] = p_own;
-        ol = T::mfmaK32(p_own, ones, ol);
+        uint32_t one2 = T::pack2(1.0f, 1.0f);
+        asm volatile("" : "+v"(one2)); // four registers for this instruction, not for the whole loop
+        ol = T::mfmaK32(p_own, make_uint4(one2, one2, one2, one2), ol);
         ldsBarrier();
 
         const int4 rescaled = lds.rescaled[half];

@@ -205,6 +205,29 @@ def test_mla_128_rows_per_workgroup(gpu_handle, oracle, monkeypatch, H, Hkv, bs,
         run_case(gpu_handle, oracle, inp, alibi=slopes, index_dtype=torch.int32)
 
 
+def both_row_block_sizes(gpu_handle, monkeypatch, inp, index_dtype=torch.int64):
+    """Outputs of the latent shape with 64 and with 128 rows per workgroup."""
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache)]
+    idx = [t.to(index_dtype).to(DEV) for t in (inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    got = []
+    for groups in ("1", "2"):
+        monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
+        out = torch.full((*inp.q.shape[:-1], 512), SENTINEL, dtype=inp.q.dtype, device=DEV)
+        got.append(run_paged_attention_prefill(gpu_handle, *dev, *idx, inp.scale, out=out).cpu())
+    return got
+
+
+@pytest.mark.parametrize("idx", [torch.int64, torch.int32, torch.uint32])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("H,bs", [(16, 16), (5, 8), (128, 64)])
+def test_mla_row_block_sizes_agree_bit_for_bit(gpu_handle, monkeypatch, H, bs, dtype, idx):
+    """Both kernels of the latent shape add the same products in the same order and round at the same places, so that the
+    rule that chooses between them decides about time alone."""
+    inp = mla_inputs(f"mla_bits_{H}_{bs}", dtype, 3, H, bs, (1, 40 if H == 128 else 200), (0, 700), seed=700 + H)
+    rows64, rows128 = both_row_block_sizes(gpu_handle, monkeypatch, inp, idx)
+    assert torch.equal(rows64, rows128), (rows64.float() - rows128.float()).abs().max()
+
+
 # ---- heads of 576 with values of 576 (the decode test list of the reference has the shape,
 # test/infiniop/paged_attention.py:106): the matrix-core kernel of the latent shape with 36 value blocks -------------
 
