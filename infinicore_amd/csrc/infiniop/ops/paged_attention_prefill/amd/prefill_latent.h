@@ -17,7 +17,7 @@
 // wavefronts per SIMD, and 56 for everything else: nothing of the loop is in scratch memory (a reload there waits for the
 // direct loads in flight too: with one query operand reloaded behind them the case below took 1 287 us).
 // Measured (16 sequences, 16 heads, 128 - 512 new tokens over 1 024 - 8 192 of history, bf16; the kernels in turn on
-// one GPU): 1 391 -> 1 006 us (589 -> 814 TFLOP/s); with K in one run of 72 chunks per row, whose reads meet in the banks two at a time, 1 270 us.
+// one GPU): 1 308 -> 995 us (626 -> 823 TFLOP/s); with K in one run of 72 chunks per row, whose reads meet in the banks two at a time, 1 270 us.
 // By the counts above LDS is the longest of the pipes: the K operands, read once per 16 rows, are three quarters of it.
 // Everything else (block search, page ids, LDS layouts, masks, lazy reference point) is as in
 // prefill_tiled.h.
@@ -41,6 +41,7 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
     constexpr int kTileChunksK = kTileTokens * G::kChunksPerRowK, kTileChunksV = kTileTokens * G::kChunksPerRowV;
     constexpr int kWaves = kLatentThreads / 64;
     constexpr int kCols = G::kColsV / 4; // blocks of 16 value columns of a wavefront
+    constexpr int kAdds = 0, kRescales = 1, kUnseen = 2;
     struct Shared {
         // K of a 16-token tile: columns 0..511 of the 16 rows, then columns 512..575 of the 16 rows; a row's 16-byte chunks
         // XOR-swizzled by the row (sixteen at a time; the last eight by half the row), so that 16 lanes that read one
@@ -51,7 +52,7 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
         uint4 v[2][2 * kTileChunksV]; // layout as in prefillTiledKernel
         uint4 p[kWaves][64];        // probabilities of 16 rows x 32 tokens, as the lanes of P.V take them
         float4 alpha[kWaves][4];    // factors by which the accumulators of the 16 rows are rescaled this step
-        int4 rescaled[kWaves / 4];  // ... and whether they are, per group of 16 rows
+        int4 update[kWaves / 4];    // ... and what the step does to them, per group of 16 rows: kAdds, kRescales or kUnseen
         float4 denominator[kWaves][4];
     };
     __shared__ Shared lds;
@@ -237,6 +238,9 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
     const int k_first = 64 * c + (g ^ c), k_last = 64 * 16 + 8 * c + (g ^ (c >> 1));
     const float unit = a.scale_log2;
     const float lazy = kLazyLog2 / unit;
+    // what the last of the wavefront's rows sees, which is the most any of them does (0 if it has no rows)
+    const int wave_row0 = block_row0 + 16 * w;
+    const int wave_sees = __builtin_amdgcn_readfirstlane(wave_row0 < total_rows ? visibleTokens(span, min(wave_row0 + 15, last_row) / a.group) : 0);
 
     auto computeStep = [&](int buf, int t0) {
         f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
@@ -300,16 +304,18 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
             const float alpha = m_new > m ? fastExp2((m - m_new) * unit) : 1.0f;
             m = m_new;
             shift = m_new == -INFINITY ? 0.0f : -m_new * unit;
-            if (g == 0) {
-                reinterpret_cast<float *>(&lds.alpha[w][0])[c] = alpha;
+            int own = lane; // addresses formed where they are used, as in loadStage
+            asm volatile("" : "+v"(own));
+            if (own < 16) {
+                reinterpret_cast<float *>(&lds.alpha[w][0])[own] = alpha;
             }
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
-                ol[rr] *= __shfl(alpha, 4 * g + rr, 64);
+                ol[rr] *= __shfl(alpha, 4 * (own >> 4) + rr, 64);
             }
         }
         if (lane == 0) {
-            reinterpret_cast<int *>(lds.rescaled)[w] = moves ? 1 : 0;
+            reinterpret_cast<int *>(lds.update)[w] = t0 >= wave_sees ? kUnseen : moves ? kRescales : kAdds;
         }
         uint32_t wds[4];
 #pragma unroll
@@ -325,12 +331,15 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
         ol = T::mfmaK32(p_own, make_uint4(one2, one2, one2, one2), ol);
         ldsBarrier();
 
-        const int4 rescaled = lds.rescaled[half];
+        const int4 update_lanes = lds.update[half];
+        const int update[4] = {__builtin_amdgcn_readfirstlane(update_lanes.x), __builtin_amdgcn_readfirstlane(update_lanes.y),
+                               __builtin_amdgcn_readfirstlane(update_lanes.z), __builtin_amdgcn_readfirstlane(update_lanes.w)};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int flag = i == 0 ? rescaled.x : i == 1 ? rescaled.y : i == 2 ? rescaled.z : rescaled.w;
-            if (__builtin_amdgcn_readfirstlane(flag) != 0) {
-                const float4 f = lds.alpha[4 * half + i][g];
+            if (__builtin_expect(update[i] == kRescales, 0)) {
+                int own = lane;
+                asm volatile("" : "+v"(own));
+                const float4 f = lds.alpha[4 * half + i][own >> 4];
 #pragma unroll
                 for (int e = 0; e < kCols; ++e) {
                     o[i][e][0] *= f.x;
@@ -351,24 +360,28 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
             const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<LdsPiece>(base + kTileChunksV * 16)));
             return make_uint4(lo.x, lo.y, hi.x, hi.y);
         };
-        constexpr int kAheadV = 2; // an operand lasts four matrix instructions here
-        uint4 vf[kAheadV];
+        // Two columns at a time, the next two requested before them; an operand lasts four matrix instructions. Rows that see
+        // nothing of the step leave it out: their probabilities are zeros, but 0 * inf is NaN, and V may hold anything at
+        // tokens that come after theirs.
+        uint4 vf[2];
 #pragma unroll
-        for (int i = 0; i < kAheadV; ++i) {
+        for (int i = 0; i < 2; ++i) {
             vf[i] = readV(i);
         }
 #pragma unroll
-        for (int e = 0; e < kCols; ++e) {
-            const uint4 cur = vf[e % kAheadV];
-            if (e + kAheadV < kCols) {
-                vf[e % kAheadV] = readV(e + kAheadV);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        for (int e = 0; e < kCols; e += 2) {
+            const uint4 cur[2] = {vf[0], vf[1]};
+            if (e + 2 < kCols) {
+                vf[0] = readV(e + 2);
+                vf[1] = readV(e + 3);
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                o[i][e] = T::mfmaK32(p_op[i], cur, o[i][e]);
+                if (__builtin_expect(update[i] != kUnseen, 1)) {
+                    o[i][e] = T::mfmaK32(p_op[i], cur[0], o[i][e]);
+                    o[i][e + 1] = T::mfmaK32(p_op[i], cur[1], o[i][e + 1]);
+                }
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
         }
     };
 

@@ -228,6 +228,27 @@ def test_mla_row_block_sizes_agree_bit_for_bit(gpu_handle, monkeypatch, H, bs, d
     assert torch.equal(rows64, rows128), (rows64.float() - rows128.float()).abs().max()
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,new,history,position", [
+    (1, 200, 0, 127),   # 128 tokens per block of 128 rows: the last of the first block
+    (1, 200, 0, 199),   # the last of a block that is not full
+    (16, 40, 3, 33),    # 8 tokens per block, the fourth of them at positions 27..34: a step of 32 tokens begins inside
+])
+def test_mla_non_finite_values_of_later_tokens(gpu_handle, monkeypatch, H, new, history, position, value):
+    """0 * inf is NaN, so a value that is not finite reaches the rows that multiply it by a probability of zero. Those are
+    the 16 rows of a wavefront that takes the step of 32 tokens it lies in, with 128 rows per workgroup as with 64; rows
+    whose wavefront sees nothing of that step keep the result of a clean cache."""
+    inp = mla_inputs("mla_non_finite", torch.bfloat16, 1, H, 16, (new, new), (history, history), seed=740 + H)
+    _, clean = both_row_block_sizes(gpu_handle, monkeypatch, inp)
+    inp.v_cache[int(inp.block_tables[0, position // 16]), :, position % 16, ::3] = value
+    rows64, rows128 = both_row_block_sizes(gpu_handle, monkeypatch, inp)
+    rows64, rows128, clean = (x.reshape(new * H, 512) for x in (rows64, rows128, clean))
+    unseen = (position // 32 * 32 - history) * H // 16 * 16  # rows of the wavefronts that end before the step
+    assert unseen > 0 and torch.equal(rows128[:unseen], clean[:unseen])
+    assert torch.equal(rows64.isnan(), rows128.isnan())
+    assert torch.allclose(rows64.nan_to_num(0.0), rows128.nan_to_num(0.0), atol=1e-2, rtol=2e-3)
+
+
 # ---- heads of 576 with values of 576 (the decode test list of the reference has the shape,
 # test/infiniop/paged_attention.py:106): the matrix-core kernel of the latent shape with 36 value blocks -------------
 
