@@ -9,9 +9,8 @@
 #include "prefill_common.h"
 #include "prefill_generic.h"
 #include "prefill_latent.h"
+#include "prefill_plan.h"
 #include "prefill_tiled.h"
-#include <cstdlib>
-#include <cstring>
 
 namespace op::paged_attention_prefill::amd {
 
@@ -22,81 +21,6 @@ using op::paged_attention::amd::Half;
 using op::paged_attention::amd::IndexI32;
 using op::paged_attention::amd::IndexI64;
 using op::paged_attention::amd::IndexU32;
-
-// Decided once, at descriptor creation, from shapes and the device alone (sequence lengths live in
-// device memory and are never read on the host).
-struct Plan {
-    bool tiled;          // matrix-core kernel (head 64 / 128 / 192 / 256 or keys 576 with values 512 / 576, power-of-two pages >= 8, 16-byte aligned strides)
-    int groups_per_wave; // tiled: R = 1 or 2 column groups per wavefront -> 64 R rows per workgroup
-    int dims_per_lane;   // element-wise kernel: ceil(max(head_size, value_size) / 64)
-};
-
-bool multipleOf8(ptrdiff_t x) { return (x % 8) == 0; }
-
-Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev) {
-    Plan plan{};
-    const long long bs = static_cast<long long>(in.page_block_size);
-    const bool pow2_page = bs >= 8 && (bs & (bs - 1)) == 0;
-    const long long group = static_cast<long long>(in.num_heads / in.num_kv_heads);
-    const long long rows = static_cast<long long>(in.total_q_tokens) * group; // per KV head
-    const bool equal_sizes = in.value_size == in.head_size
-                          && (in.head_size == 64 || in.head_size == 128 || in.head_size == 192 || in.head_size == 256);
-    // keys 576 with values 512 (latent attention) or 576 (a shape of the reference's decode tests,
-    // test/infiniop/paged_attention.py:106, taken here as well so that prompt and decode run the same class of kernel)
-    const bool latent = in.head_size == 576 && (in.value_size == 512 || in.value_size == 576);
-    plan.tiled = (equal_sizes || latent) && pow2_page
-              && multipleOf8(in.q_stride) && multipleOf8(in.q_head_stride) && multipleOf8(in.o_stride)
-              && multipleOf8(in.o_head_stride) && multipleOf8(in.k_batch_stride) && multipleOf8(in.k_head_stride)
-              && multipleOf8(in.k_row_stride) && multipleOf8(in.v_batch_stride) && multipleOf8(in.v_head_stride)
-              && multipleOf8(in.v_row_stride) && in.num_blocks > 0 && in.num_blocks <= 0x7fffffff
-              && rows < (1LL << 30) && (rows / 64 + static_cast<long long>(in.num_seqs)) * static_cast<long long>(in.num_kv_heads) < (1LL << 31)
-              // lane offsets inside a tile (15 rows + one row of bytes) are kept in 32 bits
-              && in.k_row_stride > 0 && in.k_row_stride < (1 << 26) && in.v_row_stride > 0 && in.v_row_stride < (1 << 26)
-              && static_cast<long long>(in.max_num_blocks_per_seq) * bs < (1LL << 30);
-    if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_KERNEL")) {
-        if (std::strcmp(env, "generic") == 0) {
-            plan.tiled = false;
-        }
-    }
-    // Rows per workgroup: 128 (two column groups per wavefront: every K / V operand read from LDS then feeds two
-    // matrix instructions) unless the average sequence fills no more than 64, or the batch is too small to give
-    // every compute unit as many workgroups of 128 as it holds at a time: two up to head 128, one above (there the
-    // accumulators of 128 rows need more than half the register file).
-    const long long seqs = in.num_seqs > 0 ? static_cast<long long>(in.num_seqs) : 1;
-    const long long rows_per_seq = rows / seqs;
-    const long long resident = in.head_size <= 128 ? 2 : 1;
-    int r = 2;
-    if (rows_per_seq <= 64 || rows / 128 * static_cast<long long>(in.num_kv_heads) < resident * dev.compute_units) {
-        r = 1;
-    }
-    if (latent) {
-        // Latent attention: one workgroup per compute unit with either kernel, and a round of 128-row workgroups
-        // (prefill_latent.h) takes 1.4 x as long as a round of 64-row ones (kv 2 200, 16 heads: 164 us against 119 us).
-        // So 128 rows where they save more than a third of the rounds. Measured, 64 rows against 128, by 64-row blocks:
-        // 256 (one round either way) 119 / 164 us, 300 202 / 166, 512 228 / 189, 520 (3 rounds / 2) 290 / 299,
-        // 770 407 / 343, 1 100 571 / 480; 400 sequences of 8 new tokens 342 / 244.
-        const long long units = dev.compute_units > 0 ? dev.compute_units : 1;
-        const long long streams = seqs * static_cast<long long>(in.num_kv_heads);
-        const long long rounds64 = (streams * ((rows_per_seq + 63) / 64) + units - 1) / units;
-        const long long rounds128 = (streams * ((rows_per_seq + 127) / 128) + units - 1) / units;
-        r = 2 * rounds64 > 3 * rounds128 ? 2 : 1;
-    }
-    if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_GROUPS")) {
-        const int forced = std::atoi(env);
-        if (forced == 1 || forced == 2) {
-            r = forced;
-        }
-    }
-    if (latent && (in.value_size != 512 || in.has_alibi || !(in.scale > 0.0f))) {
-        // 128 rows have a kernel of their own (prefill_latent.h) for values of 512 without ALiBi only, whatever the
-        // knob says (grid and kernel must agree on the rows per workgroup)
-        r = 1;
-    }
-    plan.groups_per_wave = r;
-    const size_t widest = in.head_size > in.value_size ? in.head_size : in.value_size;
-    plan.dims_per_lane = static_cast<int>((widest + 63) / 64);
-    return plan;
-}
 
 template <typename T, typename Tindex>
 void launchGeneric(const PrefillArgs &a, const Plan &plan, hipStream_t stream) {
