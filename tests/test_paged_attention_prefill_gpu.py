@@ -141,12 +141,14 @@ def test_mla_page_sizes_alibi_and_int32(gpu_handle, oracle, bs):
     run_case(gpu_handle, oracle, inp, alibi=slopes, index_dtype=torch.int32)
 
 
-@pytest.mark.parametrize("kernel", ["tiled", "generic"])
+@pytest.mark.parametrize("kernel", ["tiled", "tiled-2", "generic"])
 def test_mla_values_as_a_view_of_the_keys(gpu_handle, oracle, monkeypatch, kernel):
     """The latent layout of DeepSeek-style caches: one tensor of 576 columns per token, the values being its first
     512 columns (a V row stride of 576 elements)."""
     if kernel == "generic":
         monkeypatch.setenv("INFINIOP_AMD_PREFILL_KERNEL", "generic")
+    elif kernel == "tiled-2":
+        monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", "2")
     inp = mla_inputs(f"mla_view_{kernel}", torch.bfloat16, 3, 16, 16, (1, 40), (0, 150), seed=560)
     k_dev = inp.k_cache.to(DEV)
     v_dev = k_dev[..., :512]
@@ -157,9 +159,11 @@ def test_mla_values_as_a_view_of_the_keys(gpu_handle, oracle, monkeypatch, kerne
     assert_close(got, want, f"mla_view_{kernel}", want_f32)
 
 
-def test_mla_column_layout_and_garbage(gpu_handle, oracle):
+@pytest.mark.parametrize("groups", ["1", "2"])
+def test_mla_column_layout_and_garbage(gpu_handle, oracle, monkeypatch, groups):
     """V with a distinct constant per column makes the expected output that constant (every one of the 512 output
     columns lands where it belongs); NaN beyond the sequences must not leak in."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
     inp = mla_inputs("mla_cols", torch.float16, 3, 16, 16, (5, 90), (3, 200), seed=540)
     cfg = inp.config
     ramp = ((torch.arange(512, dtype=torch.float32) - 256) / 16).to(torch.float16)
@@ -182,7 +186,9 @@ def test_mla_column_layout_and_garbage(gpu_handle, oracle):
     (16, 1, 16, (8, 9), (23, 24)),      # exactly 128 rows and 144; kv lengths 31..33: one step, one token into the next
     (5, 1, 8, (1, 150), (0, 300)),      # pages of 8: two per tile; rows of a token split over row blocks
     (20, 2, 32, (1, 150), (0, 300)),
-    (16, 1, 64, (60, 200), (1000, 2300)),  # more than 64 table entries of 16 tokens, many steps
+    (16, 1, 64, (60, 200), (1000, 2300)),  # many steps
+    (16, 1, 16, (60, 200), (1000, 2300)),  # page ids from two batches of 64 table entries
+    (5, 1, 8, (60, 200), (1000, 2300)),    # from five; the two tiles of a step change batches in different steps
 ])
 def test_mla_128_rows_per_workgroup(gpu_handle, oracle, monkeypatch, H, Hkv, bs, new, history, dtype):
     """The eight-wavefront kernel of the latent shape on scores that climb (every wavefront rescales in its own steps),
@@ -190,6 +196,7 @@ def test_mla_128_rows_per_workgroup(gpu_handle, oracle, monkeypatch, H, Hkv, bs,
     monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", "2")
     inp = workloads.make_prefill_inputs(prefill_config(f"mla128_{H}_{bs}", dtype, 3, H, Hkv, 576, bs, new, history, seed=570 + bs))
     inp.v_cache = inp.v_cache[..., :512].contiguous()
+    assert history[1] < 1000 or inp.block_tables.shape[1] > {8: 256, 16: 64, 64: 32}[bs]
     for s in range(3):
         L = int(inp.seq_lens[s])
         if L % bs:
@@ -226,6 +233,51 @@ def test_mla_row_block_sizes_agree_bit_for_bit(gpu_handle, monkeypatch, H, bs, d
     inp = mla_inputs(f"mla_bits_{H}_{bs}", dtype, 3, H, bs, (1, 40 if H == 128 else 200), (0, 700), seed=700 + H)
     rows64, rows128 = both_row_block_sizes(gpu_handle, monkeypatch, inp, idx)
     assert torch.equal(rows64, rows128), (rows64.float() - rows128.float()).abs().max()
+
+
+def test_mla_128_rows_by_the_plan(gpu_handle, oracle, monkeypatch, tmp_path):
+    """No knob: a batch of more sequences than a wavefront looks through at a time, large enough for the plan to take 128
+    rows (q and out with a gap between heads), against the oracle and the 64-row kernel."""
+    from test_prefill_plan import build_probe
+    inp = mla_inputs("mla_plan", torch.bfloat16, 400, 16, 16, (7, 8), (0, 60), seed=720)
+    monkeypatch.delenv("INFINIOP_AMD_PREFILL_GROUPS", raising=False)
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    assert build_probe(tmp_path)(400, inp.q.shape[0], inp.block_tables.shape[1] * 16, units=units) == 2
+    T = inp.q.shape[0]
+    q_big = torch.zeros(T, 16, 584, dtype=torch.bfloat16, device=DEV)
+    q_big[..., :576] = inp.q.to(DEV)
+    out_big = torch.full((T, 16, 520), SENTINEL, dtype=torch.bfloat16, device=DEV)
+    rest = [t.to(DEV) for t in (inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    got = run_paged_attention_prefill(gpu_handle, q_big[..., :576], *rest, inp.scale, out=out_big[..., :512]).cpu()
+    rows = list(range(0, T, 17)) + [T - 1]
+    want, want_f32 = oracle.paged_attention_prefill(
+        inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q, inp.scale, rows=rows,
+        num_threads=ORACLE_THREADS, return_fp32=True)
+    assert_close(got[rows], want[rows], "mla_plan", want_f32[rows])
+    assert (out_big[..., 512:] == SENTINEL).all()
+    rows64, rows128 = both_row_block_sizes(gpu_handle, monkeypatch, inp)
+    assert torch.equal(rows64, got) and torch.equal(rows128, got)
+
+
+@pytest.mark.parametrize("groups", ["1", "2"])
+def test_mla_rows_nobody_owns_negative_history_and_empty_sequences(gpu_handle, oracle, monkeypatch, groups):
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
+    inp = mla_inputs("mla_edges", torch.float16, 4, 16, 16, (5, 60), (0, 80), seed=67)
+    cum = inp.cum_seq_lens_q.tolist()
+    # three extra rows past cum[-1]; sequence 1 shorter than its new tokens (its first rows see nothing, its first block of
+    # eight tokens half of that); an empty sequence inserted between 2 and 3
+    inp.q = torch.cat([inp.q, torch.randn(3, 16, 576).half()])
+    new1 = cum[2] - cum[1]
+    inp.seq_lens = inp.seq_lens.clone()
+    inp.seq_lens[1] = new1 - 4
+    inp.seq_lens = torch.cat([inp.seq_lens[:3], torch.tensor([9]), inp.seq_lens[3:]])
+    inp.cum_seq_lens_q = torch.tensor(cum[:4] + [cum[3]] + cum[4:])
+    inp.block_tables = torch.cat([inp.block_tables[:3], inp.block_tables[:1], inp.block_tables[3:]])
+    got, want = run_case(gpu_handle, oracle, inp)
+    T = cum[-1]
+    assert (got[T:] == SENTINEL).all() and (want[T:] == SENTINEL).all()
+    assert (got[cum[1]:cum[1] + 4] == SENTINEL).all()
+    assert not (got[cum[1] + 4] == SENTINEL).all()
 
 
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])

@@ -10,10 +10,9 @@ import pytest
 ROOT = Path(__file__).resolve().parents[1]
 
 
-@pytest.fixture(scope="module")
-def probe(tmp_path_factory):
+def build_probe(directory):
     """Compiles tests/prefill_plan_probe.cc with the host compiler; returns groups(num_seqs, tokens, ...) -> 1 or 2."""
-    out = tmp_path_factory.mktemp("plan") / "libprefillplanprobe.so"
+    out = directory / "libprefillplanprobe.so"
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{ROOT / 'include'}",
                     f"-I{ROOT / 'infinicore_amd' / 'csrc'}", str(ROOT / "tests" / "prefill_plan_probe.cc"), "-o", str(out)],
                    check=True, capture_output=True, text=True)
@@ -25,6 +24,11 @@ def probe(tmp_path_factory):
         return lib.latentPrefillProbe(args, scale)
 
     return groups
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    return build_probe(tmp_path_factory.mktemp("plan"))
 
 
 @pytest.fixture(autouse=True)
