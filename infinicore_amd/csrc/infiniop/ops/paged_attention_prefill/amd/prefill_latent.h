@@ -1,9 +1,11 @@
 // Prefill kernel for latent attention (keys of 576, values of 512 elements), 128 rows per workgroup, on gfx950.
 //
-// What bounds the four-wavefront kernel of prefill_tiled.h at these sizes: a wavefront there owns 16 rows, so every K
+// What the four-wavefront kernel of prefill_tiled.h pays at these sizes: a wavefront there owns 16 rows, so every K
 // and V operand read from LDS feeds one matrix instruction, and all four wavefronts read all of both tiles: 272 KiB
 // of LDS reads (2 176 clocks at 128 bytes per clock) against 1 104 clocks of matrix instructions per step of 32 tokens
-// and 64 rows; and a compute unit takes one direct load of 1 KiB every ~15 ns, 68 of them per step.
+// and 64 rows; a compute unit takes one direct load of 1 KiB every ~15 ns, 68 of them per step; and its registers
+// leave one wavefront per SIMD, with nothing to run beside it (matrix units busy 30 % of their clocks, LDS 44 %, a vector
+// instruction beside 0.3 % of the matrix clocks).
 //
 // Here one workgroup of eight wavefronts (two per SIMD) takes 128 rows, which halves the loads per row, and splits
 // the two products differently:
@@ -17,10 +19,11 @@
 // wavefronts per SIMD, and 56 for everything else: nothing of the loop is in scratch memory (a reload there waits for the
 // direct loads in flight too: with one query operand reloaded behind them the case below took 1 287 us).
 // Measured (16 sequences, 16 heads, 128 - 512 new tokens over 1 024 - 8 192 of history, bf16; the kernels in turn on
-// one GPU): 1 308 -> 995 us (626 -> 823 TFLOP/s); with K in one run of 72 chunks per row, whose reads meet in the banks two at a time, 1 270 us.
-// By the counts above LDS is the longest of the pipes: the K operands, read once per 16 rows, are three quarters of it.
-// Everything else (block search, page ids, LDS layouts, masks, lazy reference point) is as in
-// prefill_tiled.h.
+// one GPU): 1 265 -> 961 us (647 -> 852 TFLOP/s); 1 308 -> 995 on another. Neither pipe bounds it: matrix units and LDS are
+// each busy 37 % of their clocks, a vector instruction beside 16 % of the matrix clocks, 1.66 of the two wavefronts of a
+// SIMD present on average (the last round of workgroups). All eight wavefronts pass two barriers per step in the same
+// phase, so that K.Q^T (LDS), the softmax and P.V (matrix) follow one another.
+// Everything else (block search, page ids, layout of V in LDS, masks, lazy reference point) is as in prefill_tiled.h.
 #ifndef INFINICORE_AMD_PA_PREFILL_LATENT_H
 #define INFINICORE_AMD_PA_PREFILL_LATENT_H
 
@@ -45,9 +48,10 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
     struct Shared {
         // K of a 16-token tile: columns 0..511 of the 16 rows, then columns 512..575 of the 16 rows; a row's 16-byte chunks
         // XOR-swizzled by the row (sixteen at a time; the last eight by half the row), so that 16 lanes that read one
-        // chunk of the 16 rows touch all 64 banks once. (In one run of 72 chunks only eight can be swizzled, rows c and
-        // c + 8 meet in the same banks and every read takes twice as long.) One load instruction brings the first 64
-        // chunks of one row, or the last eight of eight rows, and its lane offsets cost one exclusive-or.
+        // chunk of the 16 rows touch all 64 banks once. One load instruction brings the first 64 chunks of one row, or
+        // the last eight of eight rows, and its lane offsets cost one exclusive-or. (In one run of 72 chunks as in
+        // prefillTiledKernel, only eight of them swizzled and a load across two rows: 1 270 against 1 034 us. Bank conflicts
+        // are not the reason: the counter reads the same with both kernels, the two-byte stores of the epilogue.)
         uint4 k[2][2 * kTileChunksK];
         uint4 v[2][2 * kTileChunksV]; // layout as in prefillTiledKernel
         uint4 p[kWaves][64];        // probabilities of 16 rows x 32 tokens, as the lanes of P.V take them

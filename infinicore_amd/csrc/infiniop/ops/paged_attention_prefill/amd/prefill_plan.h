@@ -16,7 +16,7 @@ namespace op::paged_attention_prefill::amd {
 // device memory and are never read on the host).
 struct Plan {
     bool tiled;          // matrix-core kernel (head 64 / 128 / 192 / 256 or keys 576 with values 512 / 576, power-of-two pages >= 8, 16-byte aligned strides)
-    int groups_per_wave; // tiled: R = 1 or 2 column groups per wavefront -> 64 R rows per workgroup
+    int groups_per_wave; // tiled: R = 1 or 2 -> 64 R rows per workgroup (R column groups of each of four wavefronts; latent attention with R = 2: one of each of eight)
     int dims_per_lane;   // element-wise kernel: ceil(max(head_size, value_size) / 64)
 };
 

@@ -1,6 +1,6 @@
 // Tiled prefill kernel on gfx950 (CDNA4, 64-lane wavefronts) for head_size = value_size = 64, 128, 192 or 256 and
-// for latent attention (keys of 576, values of 512 elements; batches that fill the chip with 128-row
-// workgroups take prefill_latent.h instead). Figures below are for head 128; the geometry per
+// for latent attention (keys of 576, values of 512 elements; where prefill_plan.h chooses 128 rows per
+// workgroup, prefill_latent.h instead). Figures below are for head 128; the geometry per
 // size is PrefillGeometry below.
 //
 // Work unit: one 256-thread workgroup = 64*R "rows" of one (sequence, KV head). A row is a (new
