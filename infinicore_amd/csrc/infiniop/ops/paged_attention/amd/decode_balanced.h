@@ -28,19 +28,6 @@ namespace op::paged_attention::amd {
 constexpr int kBalancedMinTiles = 4;   // never cut pieces finer than 64 tokens
 constexpr int kReaderSpinLimit = 1 << 22; // polls (~0.5 us each) before a reader gives up on a flag
 
-// Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS-unit permutes: this
-// runs at the head of every wavefront, before its first memory request can go out). Rows of 16 lanes are
-// scanned with row shifts, then lane 15 of rows 0 and 2 is added to the next row, then lane 31 to rows 2, 3.
-__device__ __forceinline__ int waveInclusiveSum(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false); // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false); // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false); // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false); // row_shr:8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
-    return x;
-}
-
 // Inclusive prefix sums of the per-sequence tile counts into LDS; returns the total. Executed by
 // one wavefront (lanes 0..63 of the caller).
 template <typename Tindex>

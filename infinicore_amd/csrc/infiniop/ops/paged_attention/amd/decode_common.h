@@ -152,6 +152,30 @@ __device__ __forceinline__ unsigned long long loadAgent(const unsigned long long
 __device__ __forceinline__ void waitVectorMemory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ __forceinline__ void compilerMemoryBarrier() { asm volatile("" ::: "memory"); }
 
+// Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS-unit permutes: this
+// runs at the head of every wavefront, before its first memory request can go out). Rows of 16 lanes are
+// scanned with row shifts, then lane 15 of rows 0 and 2 is added to the next row, then lane 31 to rows 2, 3.
+__device__ __forceinline__ int waveInclusiveSum(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false); // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false); // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false); // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false); // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
+// Maximum over the 64 lanes, in the same manner; every lane receives it.
+__device__ __forceinline__ int waveMaxInt(int x) {
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));
+    x = max(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
 // Sum / max over the 64 lanes of a wavefront; every lane receives the result.
 __device__ __forceinline__ float waveSum(float x) {
 #pragma unroll

@@ -364,6 +364,23 @@ def test_scores_that_climb_along_the_sequence(gpu_handle, oracle, monkeypatch, g
     inp.q[:] = (inp.q.float() * scale_rows).to(cfg.dtype)
     run_case(gpu_handle, oracle, inp)
 
+@pytest.mark.parametrize("groups", ["1", "2"])
+@pytest.mark.parametrize("seqs,heads,kv_heads", [(1, 8, 2), (7, 10, 2), (64, 4, 1), (65, 12, 4), (130, 4, 2)])
+def test_every_row_block_of_a_ragged_batch_is_worked_on(gpu_handle, oracle, monkeypatch, groups, seqs, heads, kv_heads):
+    """Blocks are dealt longest first: equal lengths, sequences without new tokens, single tokens, totals below the new
+    tokens, a group that does not divide the rows of a workgroup, more sequences than lanes."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
+    cfg = prefill_config("order", torch.float16, seqs, heads, kv_heads, 64, 16, (1, 90 if seqs > 8 else 400), (0, 300), seed=seqs)
+    inp = workloads.make_prefill_inputs(cfg)
+    new = (inp.cum_seq_lens_q[1:] - inp.cum_seq_lens_q[:-1]).clone()
+    if seqs > 1:
+        new[1] = 0
+        new[2::7] = 1
+        inp.seq_lens[3::5] = int(inp.seq_lens.min())  # equal lengths, some below the number of new tokens
+    inp.cum_seq_lens_q[1:] = torch.cumsum(new, 0)
+    inp.q = inp.q[:int(inp.cum_seq_lens_q[-1])].clone()
+    run_case(gpu_handle, oracle, inp)
+
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_element_wise_kernel_on_a_tiled_shape(gpu_handle, oracle, monkeypatch, dtype):
