@@ -43,3 +43,52 @@ def test_operators_refuse_host_tensors():
     t = torch.zeros(1, 1, 128, dtype=torch.float16)
     with pytest.raises(ValueError):
         ops.paged_attention(t, t, t, t, t)
+
+
+def test_plans_by_metadata_stream_and_thread(oracle):
+    """More shapes than the cache keeps, called again after their plans went; strided queries of one shape; several
+    threads on streams of their own at once."""
+    import threading
+
+    from infinicore_amd import ops
+
+    cfg = workloads.DecodeConfig("plans", torch.float16, 3, 8, 2, 64, 16, 200, 700, seed=5)
+    inp = workloads.make_decode_inputs(cfg)
+    q, k, v, bt, sl = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens)]
+    want = oracle.paged_attention(inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.scale).float()
+
+    def check(got):
+        assert torch.all((got.float().cpu() - want).abs() <= 1e-2 + 2e-3 * want.abs())
+
+    ops.clear_plan_cache()
+    for width in [*range(bt.shape[1], bt.shape[1] + 120), bt.shape[1]]:
+        table = torch.zeros(3, width, dtype=bt.dtype, device=DEV)
+        table[:, :bt.shape[1]] = bt
+        check(ops.paged_attention(q, k, v, table, sl, None, inp.scale))
+    assert ops._native.size() == 100
+    wide = torch.zeros(3, 8, 128, dtype=q.dtype, device=DEV)
+    wide[..., :64] = q
+    check(ops.paged_attention(wide[..., :64], k, v, bt, sl, None, inp.scale))
+
+    failures = []
+    torch.cuda.synchronize()
+
+    def work():
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(20):
+                    check(ops.paged_attention(q, k, v, bt, sl, None, inp.scale))
+        except BaseException as e:  # noqa: BLE001
+            failures.append(e)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
+    with pytest.raises(RuntimeError) as refused:
+        ops.paged_attention(q, k, v, bt, sl.to(torch.float32), None, inp.scale)
+    assert hasattr(refused.value, "status")
+    ops.clear_plan_cache()
+    assert ops._native.size() == 0
