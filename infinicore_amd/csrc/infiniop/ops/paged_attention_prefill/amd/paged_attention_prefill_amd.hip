@@ -10,6 +10,7 @@
 #include "prefill_generic.h"
 #include "prefill_latent.h"
 #include "prefill_plan.h"
+#include "prefill_split.h"
 #include "prefill_tiled.h"
 
 namespace op::paged_attention_prefill::amd {
@@ -35,13 +36,16 @@ void launchGeneric(const PrefillArgs &a, const Plan &plan, hipStream_t stream) {
 }
 
 template <typename T, typename Tindex, int KHEAD, int VHEAD, bool PLAIN>
-void launchTiledHead(const PrefillArgs &a, const Plan &plan, hipStream_t stream) {
+void launchTiledHead(const PrefillArgs &args, const Plan &plan, hipStream_t stream) {
+    PrefillArgs a = args;
     // sum over sequences of ceil(rows / block_rows) is at most floor(total rows / block_rows) + num_seqs
     const long long rows = static_cast<long long>(a.total_q_tokens) * a.group;
     const int groups = KHEAD == 576 && !PLAIN ? 1 : plan.groups_per_wave; // slopes handed over unannounced
     const int block_rows = prefillBlockRows(groups);
     static_assert(prefillBlockRows(2) == kLatentRows);
     const dim3 grid(static_cast<unsigned>((rows / block_rows + a.num_seqs) * a.num_kv_heads));
+    const int resident = groups == 2 ? prefillWorkgroupsPerUnit<KHEAD, 2>() : prefillWorkgroupsPerUnit<KHEAD, 1>();
+    a.longest_first = grid.x > static_cast<unsigned>(plan.compute_units * resident) ? 1 : 0;
     if constexpr (KHEAD == VHEAD && KHEAD <= 256) {
         if (groups == 2) {
             prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 2, PLAIN><<<grid, kPrefillThreads, 0, stream>>>(a);
@@ -53,6 +57,12 @@ void launchTiledHead(const PrefillArgs &a, const Plan &plan, hipStream_t stream)
             prefillLatentKernel<T, Tindex><<<grid, kLatentThreads, 0, stream>>>(a);
             return;
         }
+    }
+    if (a.max_parts > 1) {
+        const dim3 parts(grid.x * static_cast<unsigned>(a.max_parts));
+        prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 1, PLAIN, true><<<parts, kPrefillThreads, 0, stream>>>(a);
+        prefillMergeKernel<T, Tindex, KHEAD, VHEAD><<<dim3(grid.x, prefillBlockRows(1) / kMergeRows), kMergeThreads, 0, stream>>>(a);
+        return;
     }
     prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 1, PLAIN><<<grid, kPrefillThreads, 0, stream>>>(a);
 }
@@ -121,8 +131,9 @@ infiniStatus_t Descriptor::create(infiniopHandle_t handle, Descriptor **desc_ptr
     CHECK_RESULT(info);
     const PagedAttentionPrefillInfo in = info.take();
     const Plan plan = makePlan(in, device::amd::deviceInfo(handle->device_id));
-    // every row block keeps its softmax state in registers from the first to the last K/V token: no scratch
-    *desc_ptr = new Descriptor(new Opaque{plan}, in, 0, handle->device, handle->device_id);
+    // Scratch for the partial results of split row blocks, with 256 spare bytes to align it; 0 where none are split: a row
+    // block then keeps its softmax state in registers from the first to the last K/V token.
+    *desc_ptr = new Descriptor(new Opaque{plan}, in, plan.workspaceBytes(), handle->device, handle->device_id);
     return INFINI_STATUS_SUCCESS;
 }
 
@@ -130,12 +141,8 @@ infiniStatus_t Descriptor::calculate(void *workspace, size_t workspace_size, voi
                                      const void *k_cache, const void *v_cache, const void *block_tables,
                                      const void *seq_lens, const void *cum_seq_lens_q, const void *alibi_slopes,
                                      void *stream_) const {
-    (void)workspace;
     const PagedAttentionPrefillInfo &in = _info;
     const Plan &plan = _opaque->plan;
-    if (workspace_size < _workspace_size) {
-        return INFINI_STATUS_INSUFFICIENT_WORKSPACE;
-    }
     if (in.num_seqs == 0 || in.num_heads == 0 || in.total_q_tokens == 0) {
         return INFINI_STATUS_SUCCESS;
     }
@@ -191,6 +198,13 @@ infiniStatus_t Descriptor::calculate(void *workspace, size_t workspace_size, voi
 
     // The tiled kernel moves 16 bytes per lane; base addresses that are not 16-byte aligned take
     // the element-wise kernel instead.
+    a.max_parts = 1;
+    if (plan.max_parts > 1 && workspace != nullptr && workspace_size >= _workspace_size) {
+        char *ws = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~static_cast<uintptr_t>(255));
+        a.part_acc = reinterpret_cast<float *>(ws);
+        a.part_ml = reinterpret_cast<float2 *>(ws + plan.part_acc_bytes);
+        a.max_parts = plan.max_parts;
+    } // without the workspace it asks for, the call runs unsplit
     const bool tiled = plan.tiled && aligned16(out) && aligned16(q) && aligned16(k_cache) && aligned16(v_cache);
     auto stream = static_cast<hipStream_t>(stream_);
 

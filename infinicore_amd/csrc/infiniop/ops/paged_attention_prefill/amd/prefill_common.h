@@ -21,6 +21,11 @@ struct PrefillArgs {
     const void *kv_lens;      // [num_seqs] total K/V tokens per sequence (history + new)
     const void *cu_seqlens_q; // [num_seqs + 1] prefix sums of the new-token counts
     const float *alibi_slopes; // nullptr = no ALiBi
+    // partial results of row blocks whose tokens are split (prefill_split.h); nullptr and 1 = not split
+    float *part_acc; // [row block][KV head][part][64 rows][value_size]
+    float2 *part_ml; // [row block][KV head][part][64 rows] reference point (log2), denominator
+    int32_t max_parts;
+    int32_t longest_first; // row blocks are dealt by length (findRowBlock)
 
     float scale_log2; // scale * log2(e)
     int32_t num_seqs;

@@ -17,6 +17,10 @@ namespace op::paged_attention_prefill::amd {
 struct Plan {
     bool tiled;          // matrix-core kernel (head 64 / 128 / 192 / 256 or keys 576 with values 512 / 576, power-of-two pages >= 8, 16-byte aligned strides)
     int groups_per_wave; // tiled: R = 1 or 2 -> 64 R rows per workgroup (R column groups of each of four wavefronts; latent attention with R = 2: one of each of eight)
+    int compute_units;
+    int max_parts;       // tiled, 64 rows: workgroups that may share a row block (prefill_split.h); 1 = not split
+    size_t part_acc_bytes, part_ml_bytes; // workspace of the parts, either a multiple of 256 bytes
+    size_t workspaceBytes() const { return max_parts > 1 ? part_acc_bytes + part_ml_bytes + 256 : 0; }
     int dims_per_lane;   // element-wise kernel: ceil(max(head_size, value_size) / 64)
 };
 
@@ -52,6 +56,47 @@ inline int latentRowGroups(const PagedAttentionPrefillInfo &in, const device::am
         return seqs == 1 && 2 * history + 2 * n * (blocks - units) / blocks > 1.4 * (history + n) ? 2 : 1;
     }
     return 2 * rounds64 > 3 * rounds128 ? 2 : 1;
+}
+
+constexpr int kMaxSplitParts = 64; // the merge forms the weights of a row with a lane per part
+constexpr long long kSplitTableTokens = 128; // the shortest part (kSplitTokens of prefill_tiled.h)
+
+// How many workgroups share the tokens of a row block of 64 rows. Unsplit, a call that leaves compute units idle takes as
+// long as its longest block: `walk` microseconds for the tokens the table can hold (measured with one block per KV head
+// over 5 800 tokens). P parts take a P-th of that (1.4 times that where two of them share a unit), write and read their
+// rows back (0.9 us per MB of them) and need the merge kernel (3 us): P where the sum is smallest, among those the device
+// holds beside one another, if it takes a fifth off the walk. Measured, us unsplit / with the P this chooses / with
+// the best of 2 .. 32 (bf16; 32 / 8 heads of 128 unless said otherwise):
+//   * one sequence, 3 tokens over 600 / 5 800: 14.0 / 11.1 / 10.8, 87.7 / 14.0 / 14.2; 128 over 8 000: 130 / 34.5 / 34.5
+//   * four of 64 over 4 000: 68.8 / 36.7 / 36.2, over 500: 14.4 unsplit / 18.8; 16 of 5 over 2 000: 35.3 / 28.8 / 28.8
+//   * 16 heads of 64, 16 of 5 over 2 000 (a block per unit): 28.3 unsplit / 28.9; 28 / 4 heads of 256, one of 128 over
+//     8 000: 175 / 60.7 / 61.2; 16 latent heads, one of 3 over 5 800: 243 / 28.1 / 26.8, 16 of 5 over 2 000: 93 / 33 / 31
+inline int splitParts(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq) {
+    const long long seqs = in.num_seqs > 0 ? static_cast<long long>(in.num_seqs) : 1;
+    const long long kv_heads = static_cast<long long>(in.num_kv_heads);
+    const long long blocks = seqs * ((rows_per_seq + 63) / 64) * kv_heads;
+    const long long tokens = static_cast<long long>(in.max_num_blocks_per_seq) * static_cast<long long>(in.page_block_size);
+    const long long slots = static_cast<long long>(dev.compute_units) * (in.head_size <= 192 ? 2 : 1);
+    if (blocks <= 0) {
+        return 1;
+    }
+    const long long most = std::min(std::min(slots / blocks, (tokens + kSplitTableTokens - 1) / kSplitTableTokens),
+                                    static_cast<long long>(kMaxSplitParts));
+    const double us_per_1000 = in.head_size == 64 ? 11 : in.head_size == 128 ? 14 : in.head_size == 192 ? 22
+                             : in.head_size == 256 ? 20 : 41;
+    const double walk = us_per_1000 * 1e-3 * static_cast<double>(tokens);
+    const double row_bytes = static_cast<double>(rows_per_seq) * seqs * kv_heads * in.value_size * sizeof(float);
+    const double row_cost = 0.9e-6 * row_bytes, merge_cost = 3.0;
+    int best = 1;
+    double least = 0.8 * walk;
+    for (int p = 2; p <= most; ++p) {
+        const double shared = blocks * p > dev.compute_units && in.head_size <= 192 ? 1.4 : 1.0;
+        const double t = shared * walk / p + row_cost * p + merge_cost;
+        if (t < least) {
+            best = p, least = t;
+        }
+    }
+    return best;
 }
 
 inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev) {
@@ -105,6 +150,24 @@ inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::Dev
         r = 1;
     }
     plan.groups_per_wave = r;
+    plan.compute_units = dev.compute_units;
+    // (a forced number of rows asks for those kernels as they are)
+    const bool rows_forced = std::getenv("INFINIOP_AMD_PREFILL_GROUPS") != nullptr;
+    plan.max_parts = plan.tiled && r == 1 && !rows_forced ? splitParts(in, dev, rows_per_seq) : 1;
+    if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_PARTS")) {
+        const int forced = std::atoi(env);
+        if (plan.tiled && r == 1 && forced >= 1 && forced <= kMaxSplitParts) {
+            plan.max_parts = forced;
+        }
+    }
+    if (plan.max_parts > 1) {
+        const size_t part_rows = static_cast<size_t>(rows / 64 + seqs) * in.num_kv_heads * static_cast<size_t>(plan.max_parts) * 64;
+        if (part_rows >= (size_t{1} << 31)) { // a knob's doing: more workgroups than a launch has
+            plan.max_parts = 1;
+        }
+        plan.part_acc_bytes = part_rows * in.value_size * sizeof(float);
+        plan.part_ml_bytes = part_rows * 2 * sizeof(float);
+    }
     const size_t widest = in.head_size > in.value_size ? in.head_size : in.value_size;
     plan.dims_per_lane = static_cast<int>((widest + 63) / 64);
     return plan;

@@ -103,10 +103,25 @@ __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int
             const int64_t rows = static_cast<int64_t>(span.q_len) * a.group;
             nb = rows > 0 ? static_cast<int>((rows + block_rows - 1) / block_rows) : 0;
         }
-        const int blocks = __builtin_amdgcn_readlane(waveInclusiveSum(nb), 63);
+        const int incl = waveInclusiveSum(nb);
+        const int blocks = __builtin_amdgcn_readlane(incl, 63);
         if (x >= blocks) {
             x -= blocks;
             continue;
+        }
+        auto found = [&](int at, int its_block) {
+            seq = a.num_seqs - 1 - (base + at);
+            block = its_block;
+            span_out.q_start = __builtin_amdgcn_readlane(span.q_start, at);
+            span_out.q_len = __builtin_amdgcn_readlane(span.q_len, at);
+            span_out.history = __builtin_amdgcn_readlane(span.history, at);
+            span_out.capacity = __builtin_amdgcn_readlane(span.capacity, at);
+            span_out.kv_len = __builtin_amdgcn_readlane(span.kv_len, at);
+        };
+        if (a.longest_first == 0) {
+            const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(incl > x));
+            found(at, __builtin_amdgcn_readlane(incl, at) - 1 - x);
+            return true;
         }
         const int top = span.kv_len / block_tokens; // keys top, top - 1, .., top - nb + 1
         // blocks of this lane's sequence with a key of at least `key`
@@ -128,13 +143,7 @@ __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int
         const int before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ties >> 32),
                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ties), 0u));
         const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(((ties >> lane) & 1) != 0 && before == rank));
-        seq = a.num_seqs - 1 - (base + at);
-        block = __builtin_amdgcn_readlane(nb - 1 - (top - lo), at);
-        span_out.q_start = __builtin_amdgcn_readlane(span.q_start, at);
-        span_out.q_len = __builtin_amdgcn_readlane(span.q_len, at);
-        span_out.history = __builtin_amdgcn_readlane(span.history, at);
-        span_out.capacity = __builtin_amdgcn_readlane(span.capacity, at);
-        span_out.kv_len = __builtin_amdgcn_readlane(span.kv_len, at);
+        found(at, __builtin_amdgcn_readlane(nb - 1 - (top - lo), at));
         return true;
     }
     return false;
@@ -173,10 +182,26 @@ constexpr int prefillStepTokens() { return (KHEAD <= 128 || KHEAD == 256 || (KHE
 template <int KHEAD, int R>
 constexpr int prefillWorkgroupsPerUnit() { return (KHEAD <= 128 || (KHEAD == 192 && R == 1)) ? 2 : 1; }
 
+// The steps of one row block as its parts take them (SPLIT below): `per` each, `used` parts in all, at most max_parts and
+// none shorter than kSplitTokens but the last.
+constexpr int kSplitTokens = 128;
+struct SplitSteps {
+    int per, used;
+};
+__device__ __forceinline__ SplitSteps splitSteps(int n_steps, int step_tokens, int max_parts) {
+    const int parts = min(max_parts, (n_steps * step_tokens + kSplitTokens - 1) / kSplitTokens);
+    SplitSteps s;
+    s.per = (n_steps + parts - 1) / parts;
+    s.used = (n_steps + s.per - 1) / s.per;
+    return s;
+}
+
+// SPLIT: a.max_parts workgroups per row block, each for a range of its steps (prefill_split.h).
 // PLAIN: no ALiBi and scale > 0. The running maximum is then kept in units of the raw dot product
 // (a positive scale keeps the order) and each probability costs one fused multiply-add and one exp2.
-template <typename T, typename Tindex, int KHEAD, int VHEAD, int R, bool PLAIN>
+template <typename T, typename Tindex, int KHEAD, int VHEAD, int R, bool PLAIN, bool SPLIT = false>
 __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHEAD, R>())) prefillTiledKernel(PrefillArgs a) {
+    static_assert(!SPLIT || R == 1, "partial results are laid out for blocks of 64 rows");
     using S = typename T::storage;
     using G = PrefillGeometry<KHEAD, VHEAD>;
     constexpr int BM = prefillBlockRows(R);
@@ -203,7 +228,8 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     // multiple of 8) KV heads every die works on its own heads and the row blocks resident on a die
     // at one time are neighbours that stream the same K/V through that die's L2.
     const int kv_head = blockIdx.x % a.num_kv_heads;
-    const int block_index = blockIdx.x / a.num_kv_heads;
+    const int part = SPLIT ? static_cast<int>(blockIdx.x / a.num_kv_heads) % a.max_parts : 0;
+    const int block_index = SPLIT ? blockIdx.x / a.num_kv_heads / a.max_parts : blockIdx.x / a.num_kv_heads;
 
     int seq = 0, block = 0;
     SeqSpan span;
@@ -220,7 +246,18 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     }
     // tokens that exist; rows beyond it are zeroed in V (they may hold anything, NaN included)
     const int kv_len = __builtin_amdgcn_readfirstlane(max(span.kv_len, block_visible));
-    const int n_steps = (block_visible + BN - 1) / BN;
+    const int all_steps = (block_visible + BN - 1) / BN;
+    int first_step = 0, n_steps = all_steps; // this workgroup's: [first_step, n_steps)
+    bool partial = false;                    // ... are not all of them
+    if constexpr (SPLIT) {
+        const SplitSteps split = splitSteps(all_steps, BN, a.max_parts);
+        first_step = part * split.per;
+        n_steps = min(first_step + split.per, all_steps);
+        partial = split.used > 1;
+        if (first_step >= all_steps) {
+            return;
+        }
+    }
 
     // ---- this lane's columns: row c of each of the wavefront's R column groups ----
     uint4 q_reg[R][G::kLoadsK];
@@ -276,8 +313,8 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         }
         return id;
     };
-    int id_batch = 0;
-    int ids_cur = loadIdBatch(0), ids_next = loadIdBatch(1);
+    int id_batch = SPLIT ? min((first_step * BN) >> a.block_shift, last_entry) >> 6 : 0;
+    int ids_cur = loadIdBatch(id_batch), ids_next = loadIdBatch(id_batch + 1);
     auto pageOfEntry = [&](int entry) {
         const int e = min(entry, last_entry);
         const int raw = (e >> 6) == id_batch ? __builtin_amdgcn_readlane(ids_cur, e & 63)
@@ -632,10 +669,10 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     };
 
     // ---- pipeline ----
-    loadStage(0, false);
+    loadStage(first_step, false);
     awaitStage();
     __syncthreads();
-    for (int j = 0; j < n_steps; ++j) {
+    for (int j = first_step; j < n_steps; ++j) {
         const int t0 = j * BN;
         // stage j + 1 goes into the other buffer while this step computes (everybody is past step j - 1)
         if (j + 1 < n_steps) {
@@ -653,6 +690,34 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         }
         awaitStage();
         __syncthreads();
+    }
+
+    if constexpr (SPLIT) {
+        if (partial) { // the state as it is; rows that see nothing of these steps leave m = -inf and zeros
+            const int64_t row0 = ((static_cast<int64_t>(block_index) * a.num_kv_heads + kv_head) * a.max_parts + part) * BM + 16 * w;
+            float *acc = a.part_acc + row0 * VHEAD;
+            const int rows = last_row + 1 - block_row0 - 16 * w; // of this wavefront's 16 that exist (or more, or none)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                if (4 * g + rr < rows) {
+#pragma unroll
+                    for (int e = 0; e < G::kColsV; ++e) {
+                        acc[(4 * g + rr) * VHEAD + 16 * e + c] = o[0][e][rr];
+                    }
+                }
+            }
+            float *ml = reinterpret_cast<float *>(a.part_ml + row0);
+            if (g == 0) {
+                ml[2 * c] = m[0] * unit;
+            }
+            if (c == 0) {
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) {
+                    ml[2 * (4 * g + rr) + 1] = ol[0][rr];
+                }
+            }
+            return;
+        }
     }
 
     // ---- normalise and store. A lane holds single columns (16 e + c) of its rows; the wavefront's 16 R rows pass

@@ -338,6 +338,93 @@ def test_head_576_column_layout_garbage_alibi_and_int32(gpu_handle, oracle):
     slopes = torch.tensor([2.0 ** -(i % 5 + 1) for i in range(8)], dtype=torch.float32)
     run_case(gpu_handle, oracle, inp, alibi=slopes, index_dtype=torch.int32)
 
+# ---- row blocks whose tokens several workgroups share ----------------------------------------------------------
+
+@pytest.mark.parametrize("parts", ["2", "5", "64"])
+@pytest.mark.parametrize("D,H,Hkv,bs,dtype,idx", [
+    (64, 10, 2, 8, torch.float16, torch.int64), (128, 8, 2, 16, torch.bfloat16, torch.int32),
+    (192, 6, 6, 64, torch.float16, torch.uint32), (256, 14, 2, 16, torch.bfloat16, torch.int64)])
+def test_split_row_blocks(gpu_handle, oracle, monkeypatch, D, H, Hkv, bs, dtype, idx, parts):
+    """Lengths round the shortest part (128 tokens), its multiples and a step; up to three row blocks of a sequence; a
+    sequence that holds fewer tokens than it asks for; slopes as well as none."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", parts)
+    cfg = prefill_config(f"split{parts}", dtype, 9, H, Hkv, D, bs, (1, 40), (0, 1), seed=D)
+    cfg.max_history = 1300
+    inp = workloads.make_prefill_inputs(cfg)
+    cap = inp.block_tables.shape[1] * bs
+    lens = [1, 127, 128, 129, 255, 256, 257, 640, min(cap, 1025)]
+    rng = np.random.default_rng(D)
+    pool = inp.k_cache.shape[0]
+    inp.block_tables = torch.from_numpy(rng.integers(0, pool, (9, max(-(-max(lens) // bs), 1)))).to(torch.int64)
+    inp.seq_lens = torch.tensor(lens, dtype=torch.int64)
+    run_case(gpu_handle, oracle, inp, index_dtype=idx)
+    run_case(gpu_handle, oracle, inp, alibi=torch.tensor([2.0 ** -(i % 5 + 1) for i in range(H)]), index_dtype=idx)
+
+
+@pytest.mark.parametrize("value_size", [512, 576])
+@pytest.mark.parametrize("parts", ["3", "64"])
+def test_split_row_blocks_of_latent_heads(gpu_handle, oracle, monkeypatch, parts, value_size):
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", parts)
+    cfg = workloads.PrefillConfig("split_latent", torch.bfloat16, 3, 16, 1, 576, 16, 1, 9, 100, 900, seed=9, value_size=value_size)
+    run_case(gpu_handle, oracle, workloads.make_prefill_inputs(cfg))
+
+
+def test_parts_that_a_row_sees_nothing_of_add_nothing(gpu_handle, oracle, monkeypatch):
+    """Token 512 begins a part. Of the rows of one wavefront, 480 .. 487 see nothing of it and 488 .. 495 do; V holds
+    infinities from there on, and 0 * inf is NaN."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", "64")
+    cfg = prefill_config("split_inf", torch.float16, 1, 1, 1, 128, 16, (600, 600), (24, 24), seed=3)
+    inp = workloads.make_prefill_inputs(cfg)
+    for t in range(512, 624):
+        inp.v_cache[int(inp.block_tables[0, t // 16]), 0, t % 16] = float("inf")
+    rows = [0, 100, 447, 448, 463, 479, 480, 487]
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    got = run_paged_attention_prefill(gpu_handle, *dev, inp.scale).cpu()[rows]
+    want, want_f32 = oracle.paged_attention_prefill(
+        inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q, inp.scale, rows=rows,
+        num_threads=ORACLE_THREADS, return_fp32=True)
+    assert_close(got, want[rows], "split_inf", want_f32[rows])
+
+
+def test_split_call_without_its_workspace_and_under_capture(gpu_handle, oracle):
+    """The plan's own split: the same result without the workspace (unsplit), and from a replayed graph."""
+    from infinicore_amd import ops
+
+    cfg = prefill_config("split_plan", torch.bfloat16, 2, 32, 8, 128, 16, (3, 20), (2500, 3000), seed=8)
+    inp = workloads.make_prefill_inputs(cfg)
+    got, want = run_case(gpu_handle, oracle, inp)
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    again = ops.paged_attention_prefill(*dev, None, inp.scale)
+    out = torch.empty_like(again)
+    torch.cuda.synchronize()
+    assert torch.equal(again.cpu(), got)
+    graph = torch.cuda.CUDAGraph()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ops.paged_attention_prefill(*dev, None, inp.scale, out=out)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            ops.paged_attention_prefill(*dev, None, inp.scale, out=out)
+    for _ in range(3):
+        out.zero_()
+        ops.paged_attention_prefill(*dev, None, inp.scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.cpu(), got)
+    # from C without a workspace
+    import ctypes
+
+    from infinicore_amd import libinfiniop as L
+    plan = ops._make_paged_attention_prefill(inp.scale, out, *dev, None)
+    assert plan.workspace_bytes > 0
+    out.zero_()
+    L.check_error(L.LIBINFINIOP.infiniopPagedAttentionPrefill(
+        plan.descriptor, None, 0, *(ctypes.c_void_p(t.data_ptr()) for t in (out, *dev)), None,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    assert_close(out.cpu(), want, "no workspace")
+    plan.close()
+
 
 # ---- kernel variants --------------------------------------------------------------------------------------
 
@@ -365,9 +452,9 @@ def test_scores_that_climb_along_the_sequence(gpu_handle, oracle, monkeypatch, g
     run_case(gpu_handle, oracle, inp)
 
 @pytest.mark.parametrize("groups", ["1", "2"])
-@pytest.mark.parametrize("seqs,heads,kv_heads", [(1, 8, 2), (7, 10, 2), (64, 4, 1), (65, 12, 4), (130, 4, 2)])
+@pytest.mark.parametrize("seqs,heads,kv_heads", [(1, 8, 2), (1, 96, 96), (7, 10, 2), (9, 32, 32), (64, 4, 1), (65, 12, 4), (130, 4, 2)])
 def test_every_row_block_of_a_ragged_batch_is_worked_on(gpu_handle, oracle, monkeypatch, groups, seqs, heads, kv_heads):
-    """Blocks are dealt longest first: equal lengths, sequences without new tokens, single tokens, totals below the new
+    """Blocks are dealt longest first where there are more than 512 workgroups: equal lengths, sequences without new tokens, single tokens, totals below the new
     tokens, a group that does not divide the rows of a workgroup, more sequences than lanes."""
     monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
     cfg = prefill_config("order", torch.float16, seqs, heads, kv_heads, 64, 16, (1, 90 if seqs > 8 else 400), (0, 300), seed=seqs)
