@@ -111,6 +111,27 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
     const long long max_tiles = (max_tokens + kTileTokens - 1) / kTileTokens;
     const bool small_job = plan.tiled && !latent_head
                         && static_cast<long long>(in.num_seqs) * stream_count * max_tiles <= 64LL * dev.compute_units;
+    // Short sequences, one partition each: nothing to merge, so no second launch and no partial rows. A wavefront then walks
+    // its sequence from end to end (4.6 us and 0.024 / 0.035 / 0.045 / 0.056 us per token at head 64 / 128 / 192 / 256, alone
+    // on its SIMD); any cut costs two launches (10 us) and the time its bytes take. One partition where its walk is a tenth
+    // shorter than that, for the tokens the table can hold; up to 1 024 tokens were measured. us per call, cut as before /
+    // one partition (bf16, 32 / 8 heads, lengths from an eighth of the table up):
+    //   * head 128: 48 sequences of up to 96 11.1 / 7.2, 192 13.0 / 10.7, 512 (stays cut) 19.3 / 22.2; 128 of up to 192
+    //     20.1 / 14.5, 512 34.3 / 32.2; 256 of up to 96 24.4 / 14.7, 320 42.5 / 38.6
+    //   * head 64: 256 of up to 192 22.9 / 15.7; 128 of up to 768 28.6 / 27.1, 1 008 34.0 / 34.3 (of 806 - 1 008 46.5 / 41.5)
+    //   * head 256 with 28 / 4 heads: 128 of up to 192 24.1 / 16.4, 512 44.6 / 36.3; 48 of up to 192 (stays cut) 13.8 / 15.3
+    const double unit_tokens = static_cast<double>(units) * static_cast<double>(max_tokens);
+    const double head_cols = static_cast<double>(in.head_size);
+    // (a forced schedule asks for its cuts)
+    const bool one_partition = plan.tiled && !latent_head && std::getenv("INFINIOP_AMD_PA_SCHEDULE") == nullptr
+                            && max_tokens <= 1024 && max_tokens <= kPageIdsPerWave * bs
+                            && 4.6 + (0.0135 + 1.65e-4 * head_cols) * max_tokens < 0.9 * (10.0 + 4e-7 * head_cols * unit_tokens);
+    // From 67 MB of keys and values on (two wavefronts per SIMD in partitions of 64 tokens at head 128), small jobs are cut
+    // into 128 tokens instead of 64: half the partial rows and workgroup starts. us with 64 / 128: 32 / 8 heads of 128, 2
+    // sequences of up to 8 192 21.2 / 17.7, 8 of 500 - 2 048 15.4 / 13.9, 48 of 409 - 512 26.1 / 23.4; 28 / 4 heads of 256, 2 of
+    // up to 8 192 23.2 / 18.7, 48 of 806 - 1 008 49.7 / 47.0. Below it the walk is what counts: 16 of up to 768 with heads of
+    // 64 11.0 / 12.2, with 28 / 4 heads of 256 14.2 / 16.4.
+    const bool long_partitions = small_job && head_cols * unit_tokens >= 131072.0 * 128.0;
     // A unit of the latent-attention kernel leaves 32 KiB of partial results and advances one tile per
     // ~2 us however many units there are: fewer, longer units measured best there (more units end the
     // decode kernel sooner, but writing and merging their partial results costs more than that gains).
@@ -158,6 +179,12 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
     long long p = floorPow2(want < 1 ? 1 : want);
     const long long p_min = plan.latent_wide ? 128 : (latent_head ? 256 : 64);
     p = p < p_min ? p_min : (p > 512 ? 512 : p);
+    if (long_partitions && p < 128) {
+        p = 128;
+    }
+    if (one_partition && max_tokens > 0) {
+        p = max_tokens;
+    }
     if (const char *env = std::getenv("INFINIOP_AMD_PA_PARTITION")) {
         const int forced = std::atoi(env);
         if (forced >= 16) {
@@ -198,7 +225,7 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
     // arithmetic below divides by both counts)
     const bool can_balance = plan.tiled && !latent_head && flat_axis_fits && in.num_seqs <= static_cast<size_t>(kBalancedMaxSeqs)
                           && in.num_seqs > 0 && stream_count > 0;
-    plan.balanced = can_balance && !small_job;
+    plan.balanced = can_balance && !small_job && !one_partition;
     if (const char *env = std::getenv("INFINIOP_AMD_PA_SCHEDULE")) {
         if (std::strcmp(env, "grid") == 0) {
             plan.balanced = false;

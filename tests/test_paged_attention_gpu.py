@@ -208,6 +208,34 @@ def test_tiled_kernels_other_head_sizes(gpu_handle, oracle, monkeypatch, D, dtyp
     run_case(gpu_handle, oracle, inp)
 
 
+@pytest.mark.parametrize("D,H,Hkv,bs,table", [(64, 16, 16, 16, 1024), (64, 40, 2, 32, 96), (128, 8, 2, 16, 512),
+                                                (128, 5, 1, 128, 128), (192, 16, 2, 16, 320), (256, 14, 2, 64, 192)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_short_sequences_in_one_partition(gpu_handle, oracle, monkeypatch, dtype, D, H, Hkv, bs, table):
+    """The default plan of many short sequences: a partition as long as the table holds, no workspace; lengths round its
+    tiles, pages and end."""
+    monkeypatch.delenv("INFINIOP_AMD_PA_SCHEDULE", raising=False)
+    B = max(48, 1024 * table // 512 // Hkv)
+    cfg = custom(f"one_partition_{D}_{table}", dtype, B, H, Hkv, D, bs, 0, 40, seed=D + table, spare_block_fraction=0.1)
+    inp = workloads.make_decode_inputs(cfg)
+    rng = np.random.default_rng(table)
+    inp.block_tables = torch.from_numpy(rng.integers(0, inp.k_cache.shape[0], (B, table // bs))).to(torch.int64)
+    inp.seq_lens = torch.from_numpy(rng.integers(1, 80, B)).to(torch.int64)
+    edges = [0, 1, 15, 16, 17, 63, 64, 65, table - 17, table - 16, table - 1, table]
+    inp.seq_lens[:len(edges)] = torch.tensor(edges)
+    q, k, v, bt, sl = to_device(inp)
+    status, op = create_paged_attention(gpu_handle, torch.empty_like(q), q, k, v, bt, sl, None, inp.scale)
+    assert status == 0 and workspace_size_attention(op) == 0
+    assert L.LIBINFINIOP.infiniopDestroyPagedAttentionDescriptor(op) == 0
+    got = run_paged_attention(gpu_handle, q, k, v, bt, sl, inp.scale)
+    want, want_f32 = oracle_of(oracle, inp, return_fp32=True)
+    assert_close(got[1:], want[1:], cfg.name, want_f32[1:])
+    slopes = torch.tensor([2.0 ** -(i % 6 + 1) for i in range(H)])
+    got = run_paged_attention(gpu_handle, q, k, v, bt, sl, inp.scale, alibi=slopes.to(DEV))
+    want, want_f32 = oracle_of(oracle, inp, alibi_slopes=slopes, return_fp32=True)
+    assert_close(got[1:], want[1:], cfg.name, want_f32[1:])
+
+
 @pytest.mark.parametrize("D", [64, 192, 256])
 def test_other_head_sizes_match_the_elementwise_kernel_bit_for_bit_in_layout(gpu_handle, oracle, monkeypatch, D):
     """Every output column lands where the element-wise kernel puts it: V with a distinct constant per
