@@ -76,6 +76,8 @@ __device__ __forceinline__ uint4 loadLane16Cached(const char *uniform_base, uint
 // Rows of one workgroup for R column groups per wavefront.
 __host__ __device__ constexpr int prefillBlockRows(int r) { return 64 * r; }
 
+constexpr unsigned kLongestFirstRounds = 6; // of workgroups that the device holds at a time
+
 // Which (sequence, row block) workgroup `x` of a KV head works on: the x-th longest block of the batch. The dispatcher
 // starts workgroups in the order of their numbers, so the long blocks of a ragged batch start first and the last round
 // is made of short ones. A block's rank goes by the tokens it sees, counted in blocks of tokens (block_rows rows are
