@@ -4,20 +4,29 @@
 // a small call (us a pass, in Python / here): rotation, cache write and decode of one sequence of 1 023 tokens 26.9 / 12.6, of
 // four prompts of 19 - 250 24.1 / 16.8; a small decode alone 12.1 / 6.6; a first call with new metadata 71 / 36.
 //
-// A plan (operator descriptor and workspace) is made by a Python function the first time its metadata is seen and kept
-// in a cache bounded by least recent use; device and stream are part of the key, so a workspace serves one stream.
+// A plan (operator descriptor) is made by a Python function the first time its metadata is seen and kept in a cache
+// bounded by least recent use; device and stream are part of the key. Scratch of a call:
+//   * prefill: from torch's allocator for this call alone, given back when its kernels are enqueued, as torch's own
+//     operators do. Calls of several threads never share it, under capture it comes from the graph's pool, and a hundred
+//     plans (one per prompt shape) do not hold tens of MB each beside a KV pool that was sized without them.
+//   * decode: kept by the plan, because a call leaves in it where its first tiles were for the next call (the next layer of
+//     a step). Threads that make the same call on one stream take turns (the launches of one call would otherwise interleave
+//     with the other's between partial rows and merge). Calls under capture have a buffer from the graph's pool, one per
+//     capture, which lives as long as the graph, whatever becomes of the plan.
 // The cache is only touched with the interpreter lock held; the lock is given up during the call into the library, and a
 // shared pointer keeps the plan alive until the call is back, whoever evicts it meanwhile.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "infinicore/lru_cache.h"
@@ -34,14 +43,15 @@ struct Operator {
     int device_tensor;  // the tensor that says which device (and must be on one)
     bool has_out;       // tensors[0] is the output, allocated here where it is None
     bool last_optional; // the last tensor may be None
+    bool keeps_scratch; // its scratch is worth keeping from call to call
 };
 constexpr Operator kOperators[] = {
-    {7, 1, true, true},    // paged_attention: out, q, k_cache, v_cache, block_tables, cache_lens, alibi_slopes
-    {8, 1, true, true},    // paged_attention_prefill: ... seq_lens, cum_seq_lens_q, alibi_slopes
-    {5, 2, false, false},  // paged_caching: k_cache, v_cache, k, v, slot_mapping
-    {8, 2, false, false},  // rope_paged_caching: ... slot_mapping, pos_ids, sin_table, cos_table
-    {10, 4, false, false}, // the same with q_out, q in front
-    {5, 2, false, false},  // kv_caching: k_cache, v_cache, k, v, past_kv_lengths
+    {7, 1, true, true, true},     // paged_attention: out, q, k_cache, v_cache, block_tables, cache_lens, alibi_slopes
+    {8, 1, true, true, false},    // paged_attention_prefill: ... seq_lens, cum_seq_lens_q, alibi_slopes
+    {5, 2, false, false, false},  // paged_caching: k_cache, v_cache, k, v, slot_mapping
+    {8, 2, false, false, false},  // rope_paged_caching: ... slot_mapping, pos_ids, sin_table, cos_table
+    {10, 4, false, false, false}, // the same with q_out, q in front
+    {5, 2, false, false, false},  // kv_caching: k_cache, v_cache, k, v, past_kv_lengths
 };
 constexpr int kNumOperators = sizeof(kOperators) / sizeof(kOperators[0]);
 constexpr int kMaxTensors = 10;
@@ -59,8 +69,11 @@ std::vector<PyObject *> g_retired; // plans nobody uses any more, to be closed w
 
 struct Entry {
     PyObject *plan = nullptr;
-    void *descriptor = nullptr, *workspace = nullptr;
+    void *descriptor = nullptr;
     size_t workspace_bytes = 0;
+    std::mutex turn; // of the calls that use the buffers
+    c10::DataPtr scratch, captured_scratch;
+    unsigned long long capture = 0; // that captured_scratch belongs to
     ~Entry() {
         if (plan != nullptr) {
             g_retired.push_back(plan);
@@ -102,28 +115,46 @@ bool readPlan(PyObject *plan, Entry &entry) {
         Py_DECREF(x);
         return !PyErr_Occurred();
     };
-    unsigned long long descriptor = 0, workspace = 0, bytes = 0;
-    if (!number("descriptor_address", descriptor) || !number("workspace_address", workspace) || !number("workspace_bytes", bytes)) {
+    unsigned long long descriptor = 0, bytes = 0;
+    if (!number("descriptor_address", descriptor) || !number("workspace_bytes", bytes)) {
         return false;
     }
     entry.descriptor = reinterpret_cast<void *>(static_cast<uintptr_t>(descriptor));
-    entry.workspace = reinterpret_cast<void *>(static_cast<uintptr_t>(workspace));
     entry.workspace_bytes = static_cast<size_t>(bytes);
     entry.plan = plan; // the reference goes with it
     return true;
 }
 
-int callLibrary(int kind, const Entry &e, void *const *p, void *stream) {
+int callLibrary(int kind, const Entry &e, void *workspace, void *const *p, void *stream) {
     using V = void *;
     using C = const void *;
     void *const fn = g_library.run[kind];
     switch (kind) {
-    case 0: return reinterpret_cast<int (*)(V, V, size_t, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, e.workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], stream);
-    case 1: return reinterpret_cast<int (*)(V, V, size_t, V, C, C, C, C, C, C, C, V)>(fn)(e.descriptor, e.workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], stream);
-    case 3: return reinterpret_cast<int (*)(V, V, size_t, V, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, e.workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], stream);
-    case 4: return reinterpret_cast<int (*)(V, V, size_t, V, C, V, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, e.workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], stream);
-    default: return reinterpret_cast<int (*)(V, V, size_t, V, V, C, C, C, V)>(fn)(e.descriptor, e.workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], stream);
+    case 0: return reinterpret_cast<int (*)(V, V, size_t, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], stream);
+    case 1: return reinterpret_cast<int (*)(V, V, size_t, V, C, C, C, C, C, C, C, V)>(fn)(e.descriptor, workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], stream);
+    case 3: return reinterpret_cast<int (*)(V, V, size_t, V, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], stream);
+    case 4: return reinterpret_cast<int (*)(V, V, size_t, V, C, V, V, C, C, C, C, C, C, V)>(fn)(e.descriptor, workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], stream);
+    default: return reinterpret_cast<int (*)(V, V, size_t, V, V, C, C, C, V)>(fn)(e.descriptor, workspace, e.workspace_bytes, p[0], p[1], p[2], p[3], p[4], stream);
     }
+}
+
+struct WithoutInterpreterLock {
+    PyThreadState *const state = PyEval_SaveThread();
+    ~WithoutInterpreterLock() { PyEval_RestoreThread(state); }
+};
+
+// The capture a stream is part of; 0 where it is not capturing.
+unsigned long long captureOf(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (stream == nullptr) { // cannot be captured, and may not be asked while another stream is
+        return 0;
+    }
+    if (hipStreamGetCaptureInfo(stream, &status, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusActive ? id : 0;
 }
 
 // setup(run function addresses, address of infinirtSetDevice, device type, plans kept)
@@ -197,7 +228,7 @@ PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         allocated = at::empty(shape, at::TensorOptions().dtype(on.scalar_type()).device(on.device()));
         t[0] = &allocated;
     }
-    void *const stream = c10::hip::getCurrentHIPStream(device).stream();
+    const hipStream_t stream = c10::hip::getCurrentHIPStream(device).stream();
 
     MetaKey key;
     key.words.reserve(128);
@@ -257,12 +288,29 @@ PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     }
 
     int status;
-    PyThreadState *const state = PyEval_SaveThread();
-    status = g_library.set_device(g_library.device_type, device);
-    if (status == 0) {
-        status = callLibrary(static_cast<int>(kind), *entry, pointers, stream);
+    {
+        const WithoutInterpreterLock unlocked; // (also while an allocation waits for the device)
+        status = g_library.set_device(g_library.device_type, device);
+        const auto allocate = [&] { return c10::hip::HIPCachingAllocator::get()->allocate(entry->workspace_bytes); }; // of the current stream
+        if (status == 0 && entry->workspace_bytes == 0) {
+            status = callLibrary(static_cast<int>(kind), *entry, nullptr, pointers, stream);
+        } else if (status == 0 && !op.keeps_scratch) {
+            const c10::DataPtr scratch = allocate();
+            status = callLibrary(static_cast<int>(kind), *entry, scratch.get(), pointers, stream);
+        } else if (status == 0) {
+            const unsigned long long capture = captureOf(stream);
+            const std::lock_guard<std::mutex> lock(entry->turn);
+            c10::DataPtr &scratch = capture != 0 ? entry->captured_scratch : entry->scratch;
+            if (capture != 0 && capture != entry->capture) {
+                scratch.clear();
+                entry->capture = capture;
+            }
+            if (!scratch) {
+                scratch = allocate();
+            }
+            status = callLibrary(static_cast<int>(kind), *entry, scratch.get(), pointers, stream);
+        }
     }
-    PyEval_RestoreThread(state);
     entry.reset();
     if (!g_retired.empty()) {
         closeRetired();

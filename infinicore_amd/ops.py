@@ -71,25 +71,15 @@ def _describe(t: torch.Tensor):
 
 
 class _Plan:
-    """An operator descriptor plus its workspace; owns both until the native cache closes it. A plan belongs to one
-    stream (the stream is part of the cache key): two calls with the same shapes on different streams would
-    otherwise write their partial results into the same workspace at the same time."""
+    """An operator descriptor, until the native cache closes it, and the bytes of scratch its calls need."""
 
-    def __init__(self, descriptor, destroy, workspace_bytes: int, device: torch.device):
+    def __init__(self, descriptor, destroy, workspace_bytes: int):
         self.descriptor = descriptor
         self._destroy = destroy
         self.workspace_bytes = workspace_bytes
-        self.workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device) if workspace_bytes else None
-        self.stream = torch.cuda.current_stream(device)  # the stream of the cache key this plan is stored under
         self.descriptor_address = ctypes.cast(descriptor, c_void_p).value
-        self.workspace_address = self.workspace.data_ptr() if workspace_bytes else 0
 
     def close(self):
-        if self.workspace is not None:
-            # evicted while a kernel on the plan's stream may still be using the workspace: the caching
-            # allocator may hand the memory out again only after that stream has passed this point
-            self.workspace.record_stream(self.stream)
-            self.workspace = None
         if self.descriptor is not None:
             check_error(self._destroy(self.descriptor))
             self.descriptor = None
@@ -118,7 +108,7 @@ def _plan(create, workspace_size, destroy, device, tensors, *more, optional=None
             lib.destroy_tensor_descriptor(d)
     size = c_size_t(0)
     check_error(getattr(LIBINFINIOP, workspace_size)(op, ctypes.byref(size)))
-    return _Plan(op, getattr(LIBINFINIOP, destroy), size.value, device)
+    return _Plan(op, getattr(LIBINFINIOP, destroy), size.value)
 
 
 def _make_paged_attention(scale, *tensors):
