@@ -86,7 +86,9 @@ __INFINI_C __export infiniStatus_t infinicoreOpPlannedWorkspaceSize(infinicorePl
  *      (src/infinicore/ops/paged_attention/paged_attention.cc:38-42). Descriptor from the same cache;
  *      the workspace is the calling thread's buffer for (device, stream), which grows to the largest
  *      size asked for and is reused by every later immediate call on that stream (calls on one stream
- *      are ordered, so they can share it). Growing it allocates: not under stream capture. ---- */
+ *      are ordered, so they can share it). Growing it allocates: not under stream capture. A prefill that
+ *      is captured uses no workspace (its row blocks are then not split), so its graph depends on no
+ *      buffer of the thread's. ---- */
 __INFINI_C __export infiniStatus_t infinicoreOpPagedAttention(
     const infinicoreTensorView_t *out, const infinicoreTensorView_t *q, const infinicoreTensorView_t *k_cache,
     const infinicoreTensorView_t *v_cache, const infinicoreTensorView_t *block_tables,

@@ -6,6 +6,8 @@
 #include "infiniop.h"
 #include "lru_cache.h"
 
+#include <hip/hip_runtime_api.h>
+
 #include <array>
 #include <functional>
 #include <map>
@@ -206,9 +208,26 @@ infiniStatus_t makePlan(infinicorePlannedOp_t *plan_ptr, std::shared_ptr<Descrip
     return INFINI_STATUS_SUCCESS;
 }
 
+bool capturing(infiniDevice_t device, infinirtStream_t stream) {
+    if (device != INFINI_DEVICE_AMD || stream == nullptr) { // (the default stream cannot be captured)
+        return false;
+    }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status == hipStreamCaptureStatusActive;
+}
+
 // immediate call: the thread's workspace for (device, stream), grown when a descriptor asks for more
 infiniStatus_t runImmediate(const std::shared_ptr<Descriptor> &descriptor, infiniDevice_t device, int device_id,
-                            const CallFn &call, infinirtStream_t stream) {
+                            const CallFn &call, infinirtStream_t stream, bool runs_without_workspace) {
+    // A graph would keep the address of a buffer that a later call may replace, and nothing may be allocated now: an
+    // operator that can do without is recorded without.
+    if (runs_without_workspace && descriptor->workspace_bytes != 0 && capturing(device, stream)) {
+        return call(descriptor->desc, nullptr, 0, stream);
+    }
     Workspace &arena = state().arenas[{static_cast<int>(device), device_id, stream}];
     if (arena.bytes < descriptor->workspace_bytes) {
         if (arena.ptr != nullptr) {
@@ -227,6 +246,7 @@ struct Prepared {
     infiniDevice_t device = INFINI_DEVICE_CPU;
     int device_id = 0;
     CallFn call;
+    bool runs_without_workspace = false; // prefill: its row blocks are then not split
 };
 
 infiniStatus_t preparePagedAttention(Prepared *p, const infinicoreTensorView_t *out, const infinicoreTensorView_t *q,
@@ -299,6 +319,7 @@ infiniStatus_t preparePagedAttentionPrefill(Prepared *p, const infinicoreTensorV
     p->call = [=](InfiniopDescriptor *desc, void *ws, size_t ws_bytes, infinirtStream_t stream) {
         return infiniopPagedAttentionPrefill(desc, ws, ws_bytes, o, qd, k, v, bt, sl, cu, al, stream);
     };
+    p->runs_without_workspace = true;
     return INFINI_STATUS_SUCCESS;
 }
 
@@ -354,7 +375,7 @@ infiniStatus_t finishPlan(infinicorePlannedOp_t *plan_ptr, infiniStatus_t prepar
 
 infiniStatus_t finishImmediate(infiniStatus_t prepared, const Prepared &p, infinirtStream_t stream) {
     RETURN_IF_ERROR(prepared);
-    return runImmediate(p.descriptor, p.device, p.device_id, p.call, stream);
+    return runImmediate(p.descriptor, p.device, p.device_id, p.call, stream, p.runs_without_workspace);
 }
 
 } // namespace

@@ -216,6 +216,37 @@ def test_paged_attention_prefill_immediate_and_planned(core, oracle):
     assert core.cache_stats(core.OpKind.PAGED_ATTENTION_PREFILL) == (1, 1, 1)
 
 
+def test_captured_immediate_prefill_depends_on_no_workspace(core, oracle):
+    """A prefill that would split its row blocks, captured as the first call of its thread on the stream (nothing may be
+    allocated then), and again when the thread has a workspace: replays are right after that workspace went."""
+    print("case captured prefill", flush=True)
+    cfg = workloads.PrefillConfig("captured", torch.bfloat16, 2, 32, 8, 128, 16, 5, 5, 3000, 3000, seed=82)
+    inp = workloads.make_prefill_inputs(cfg)
+    want = oracle.paged_attention_prefill(inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens,
+                                          inp.cum_seq_lens_q, inp.scale)
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    out = torch.zeros_like(dev[0])
+    with core.PlannedOp("paged_attention_prefill", out, *dev, None, scale=inp.scale) as plan:
+        assert plan.workspace_bytes > 0
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for first in (True, False):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(side):
+            if not first:
+                core.paged_attention_prefill_(out, *dev, None, inp.scale)
+                side.synchronize()
+            with torch.cuda.graph(graph, stream=side):
+                core.paged_attention_prefill_(out, *dev, None, inp.scale)
+        core.cache_clear()  # frees the thread's workspaces
+        for _ in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert close(out, want)
+
+
 def test_strided_views_are_part_of_the_key(core, oracle):
     """A padded query (row stride larger than heads x head size) is another descriptor than the packed one."""
     inp, (q, k, v, bt, sl), want = decode_case(oracle, "strided", torch.float16, 3, 8, 8, 128, 1, 200, 80)
