@@ -47,7 +47,11 @@ __INFINI_C __export infiniStatus_t infiniopCreatePagedAttentionPrefillDescriptor
     infiniopTensorDescriptor_t alibi_slopes_desc,
     float scale);
 
-/* Bytes of device scratch the run call needs (0 on this backend).
+/* Bytes of device scratch the run call can use: 0, or, for a few new tokens over what may be a long
+ * history, room for the partial results of row blocks that several workgroups share (up to some tens of
+ * MB; any alignment, any content). A call that is handed none, or less, is still right: its blocks are
+ * then not shared, which takes several times as long where the history is long, and may differ in the
+ * last bit. Calls that overlap in time need a workspace each.
  * Replaces src/infiniop/ops/paged_attention_prefill/operator.cc:74-111. */
 __INFINI_C __export infiniStatus_t infiniopGetPagedAttentionPrefillWorkspaceSize(
     infiniopPagedAttentionPrefillDescriptor_t desc,

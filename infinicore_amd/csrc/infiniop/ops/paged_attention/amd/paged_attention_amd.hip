@@ -13,8 +13,6 @@
 #include "decode_tiled.h"
 #include "decode_mla.h"
 #include "decode_plan.h"
-#include <atomic>
-#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -159,16 +157,6 @@ infiniStatus_t launchByIndex(infiniDtype_t index_dtype, const DecodeArgs &a, con
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-// A 64-bit value no earlier call of this process has used and that is never 0 (the value of a cleared flag):
-// a counter that starts at a point of the clock, spread over the word by an odd multiplier. What a workspace
-// holds before its first use can only be mistaken for it by a 2^-64 accident.
-unsigned long long nextToken() {
-    static std::atomic<unsigned long long> counter{
-        static_cast<unsigned long long>(std::chrono::steady_clock::now().time_since_epoch().count()) | 1ull};
-    unsigned long long t = counter.fetch_add(1, std::memory_order_relaxed) * 0x9e3779b97f4a7c15ull;
-    return t != 0 ? t : 0x9e3779b97f4a7c15ull;
-}
 
 } // namespace
 
@@ -317,7 +305,7 @@ infiniStatus_t Descriptor::launch(void *workspace, void *out, const void *q, con
         a.seq_pieces = reinterpret_cast<int2 *>(ws + plan.acc_bytes + 2 * plan.ml_bytes);
         a.seg_flags = reinterpret_cast<unsigned long long *>(ws + plan.acc_bytes + 2 * plan.ml_bytes + plan.pieces_bytes);
         a.first_tiles = reinterpret_cast<int32_t *>(ws + plan.acc_bytes + 2 * plan.ml_bytes + plan.pieces_bytes + plan.flags_bytes);
-        a.token = nextToken();
+        a.token = device::amd::nextToken();
         // the 64-head latent-attention kernel plans its units per call from the actual lengths and leaves the
         // partition size it chose in the first word of the pieces region, for the merge kernel
         if (plan.latent_wide && !plan.partition_forced && in.num_seqs <= 256 && plan.tiled && aligned16(out) && aligned16(q)

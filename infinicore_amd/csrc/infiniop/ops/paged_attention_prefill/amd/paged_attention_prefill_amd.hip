@@ -10,7 +10,6 @@
 #include "prefill_generic.h"
 #include "prefill_latent.h"
 #include "prefill_plan.h"
-#include "prefill_split.h"
 #include "prefill_tiled.h"
 
 namespace op::paged_attention_prefill::amd {
@@ -60,9 +59,10 @@ void launchTiledHead(const PrefillArgs &args, const Plan &plan, hipStream_t stre
         }
     }
     if (a.max_parts > 1) {
-        const dim3 parts(grid.x * static_cast<unsigned>(a.max_parts));
-        prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 1, PLAIN, true><<<parts, kPrefillThreads, 0, stream>>>(a);
-        prefillMergeKernel<T, Tindex, KHEAD, VHEAD><<<dim3(grid.x, prefillBlockRows(1) / kMergeRows), kMergeThreads, 0, stream>>>(a);
+        a.row_blocks = static_cast<int32_t>(grid.x / static_cast<unsigned>(a.num_kv_heads));
+        a.part_workgroups = grid.x * static_cast<unsigned>(a.max_parts);
+        const dim3 all(a.part_workgroups + grid.x * static_cast<unsigned>(a.merge_workgroups));
+        prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 1, PLAIN, true><<<all, kPrefillThreads, 0, stream>>>(a);
         return;
     }
     prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 1, PLAIN><<<grid, kPrefillThreads, 0, stream>>>(a);
@@ -204,7 +204,12 @@ infiniStatus_t Descriptor::calculate(void *workspace, size_t workspace_size, voi
         char *ws = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~static_cast<uintptr_t>(255));
         a.part_acc = reinterpret_cast<float *>(ws);
         a.part_ml = reinterpret_cast<float2 *>(ws + plan.part_acc_bytes);
+        a.part_flags = reinterpret_cast<unsigned long long *>(ws + plan.part_acc_bytes + plan.part_ml_bytes);
+        a.token = device::amd::nextToken();
         a.max_parts = plan.max_parts;
+        a.merge_workgroups = plan.merge_workgroups;
+        a.split_from = plan.split_from;
+        a.part_cost = plan.part_cost;
     } // without the workspace it asks for, the call runs unsplit
     const bool tiled = plan.tiled && aligned16(out) && aligned16(q) && aligned16(k_cache) && aligned16(v_cache);
     auto stream = static_cast<hipStream_t>(stream_);

@@ -21,10 +21,6 @@ struct PrefillArgs {
     const void *kv_lens;      // [num_seqs] total K/V tokens per sequence (history + new)
     const void *cu_seqlens_q; // [num_seqs + 1] prefix sums of the new-token counts
     const float *alibi_slopes; // nullptr = no ALiBi
-    // partial results of row blocks whose tokens are split (prefill_split.h); nullptr and 1 = not split
-    float *part_acc; // [row block][KV head][part][64 rows][value_size]
-    float2 *part_ml; // [row block][KV head][part][64 rows] reference point (log2), denominator
-    int32_t max_parts;
     int32_t longest_first; // row blocks are dealt by length (findRowBlock)
 
     float scale_log2; // scale * log2(e)
@@ -46,6 +42,19 @@ struct PrefillArgs {
     int64_t k_batch_stride, k_head_stride, k_row_stride;
     int64_t v_batch_stride, v_head_stride, v_row_stride;
     int64_t block_table_batch_stride;
+
+    // Row blocks whose tokens are split (prefill_split.h); nullptr and 1 = none are. (Last: the other kernels fetch the block
+    // of arguments up to here.)
+    float *part_acc;                // [row block][KV head][part][64 rows][value_size]
+    float2 *part_ml;                // [row block][KV head][part][64 rows] reference point (log2), denominator
+    unsigned long long *part_flags; // [row block][KV head][part][64 rows] `token` once the row is there
+    unsigned long long token;       // of this call
+    int32_t row_blocks;             // an upper bound of the row blocks: the grid holds that many
+    unsigned part_workgroups;       // row_blocks x KV heads x max_parts; the workgroups that merge come behind
+    int32_t max_parts;
+    int32_t merge_workgroups; // of a row block and KV head: 1, 2, 4 or 8
+    int32_t split_from; // tokens that a row block sees, at least, to be split
+    float part_cost;    // what the rows of one more part cost, in tokens of a workgroup's walk
 };
 
 // What one sequence contributes. Query token j (0 <= j < q_len) is row q_start + j of q / out and

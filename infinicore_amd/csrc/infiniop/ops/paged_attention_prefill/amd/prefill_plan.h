@@ -18,9 +18,12 @@ struct Plan {
     bool tiled;          // matrix-core kernel (head 64 / 128 / 192 / 256 or keys 576 with values 512 / 576, power-of-two pages >= 8, 16-byte aligned strides)
     int groups_per_wave; // tiled: R = 1 or 2 -> 64 R rows per workgroup (R column groups of each of four wavefronts; latent attention with R = 2: one of each of eight)
     int compute_units;
-    int max_parts;       // tiled, 64 rows: workgroups that may share a row block (prefill_split.h); 1 = not split
-    size_t part_acc_bytes, part_ml_bytes; // workspace of the parts, either a multiple of 256 bytes
-    size_t workspaceBytes() const { return max_parts > 1 ? part_acc_bytes + part_ml_bytes + 256 : 0; }
+    int max_parts;       // tiled, 64 rows: workgroups that may share a row block (prefill_split.h); 1 = none is split
+    int merge_workgroups; // of a row block: 1, 2, 4 or 8
+    int split_from;      // tokens from which a row block is split, and what a further part costs in tokens (PrefillArgs)
+    float part_cost;
+    size_t part_acc_bytes, part_ml_bytes, part_flags_bytes; // workspace of the parts, each a multiple of 256 bytes
+    size_t workspaceBytes() const { return max_parts > 1 ? part_acc_bytes + part_ml_bytes + part_flags_bytes + 256 : 0; }
     int dims_per_lane;   // element-wise kernel: ceil(max(head_size, value_size) / 64)
 };
 
@@ -59,44 +62,64 @@ inline int latentRowGroups(const PagedAttentionPrefillInfo &in, const device::am
 }
 
 constexpr int kMaxSplitParts = 64; // the merge forms the weights of a row with a lane per part
-constexpr long long kSplitTableTokens = 128; // the shortest part (kSplitTokens of prefill_tiled.h)
+constexpr long long kSplitTableTokens = 128; // a part per that many tokens at most (kSplitTokens of prefill_split.h)
 
-// How many workgroups share the tokens of a row block of 64 rows. Unsplit, a call that leaves compute units idle takes as
-// long as its longest block: `walk` microseconds for the tokens the table can hold (measured with one block per KV head
-// over 5 800 tokens). P parts take a P-th of that (1.4 times that where two of them share a unit), write and read their
-// rows back (0.9 us per MB of them) and need the merge kernel (3 us): P where the sum is smallest, among those the device
-// holds beside one another, if it takes a fifth off the walk. Measured, us unsplit / with the P this chooses / with
-// the best of 2 .. 32 (bf16; 32 / 8 heads of 128 unless said otherwise):
-//   * one sequence, 3 tokens over 600 / 5 800: 14.0 / 11.1 / 10.8, 87.7 / 14.0 / 14.2; 128 over 8 000: 130 / 34.5 / 34.5
-//   * four of 64 over 4 000: 68.8 / 36.7 / 36.2, over 500: 14.4 unsplit / 18.8; 16 of 5 over 2 000: 35.3 / 28.8 / 28.8
-//   * 16 heads of 64, 16 of 5 over 2 000 (a block per unit): 28.3 unsplit / 28.9; 28 / 4 heads of 256, one of 128 over
-//     8 000: 175 / 60.7 / 61.2; 16 latent heads, one of 3 over 5 800: 243 / 28.1 / 26.8, 16 of 5 over 2 000: 93 / 33 / 31
-inline int splitParts(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq) {
+// How many workgroups may share the tokens of a row block of 64 rows, and what the kernel needs to settle how many do.
+// Unsplit, a call that leaves compute units idle takes as long as its longest block: `walk` microseconds for the tokens it
+// sees (measured with one block per KV head over 5 800 tokens). P parts take a P-th of that (1.4 times that where two of
+// them share a unit), 3.5 us to meet, and 0.3 us per MB of rows that they leave and that are read back. The host knows what
+// the table can hold, not the lengths: it picks the P of the longest walk (among those the device holds beside one another)
+// if that takes a fifth off it, and hands on the tokens from which a block gains at all and what a part costs, so that
+// the kernel leaves short blocks whole and cuts middling ones into fewer parts (splitSteps).
+// Measured, us (bf16; 32 / 8 heads of 128 unless said otherwise), never split / on a table as wide as the sequence / on one
+// of 32 768 tokens; in brackets the latter two with a merge kernel of its own, which was launched wherever the table was wide:
+//   * one sequence, 3 tokens over 2 000: 33.4 / 10.2 / 9.9 (12.0, 11.8); 100 over 2 000: 36.7 / 18.0 / 17.9 (20.0, 17.8),
+//     over 500: 14.8 / 14.9 / 13.9 (14.7, 14.5); four of 64 over 5 000: 82 / 44 / 42 (42, 41); 16 of 5 over 2 000: 35.4 /
+//     29.2 / 29.5 (28.5, 28.1)
+//   * 16 heads of 64, four of 64 over 2 000: 31.5 / 18.0 / 18.0 (19.6, 18.5); 28 / 4 heads of 256, one of 100 over 2 000:
+//     50.0 / 28.0 / 27.3 (28.6, 25.0); 16 latent heads, one of 3 over 2 000: 91 / 20.4 / 20.1 (20.1, 20.1), 16 of 5: 96 / 31.1 / 30.9
+//   * without history, where nothing is split and the table alone says that it might be: one of 3 tokens 5.7 / 5.8 / 6.8
+//     (6.2, 9.7), one of 100 7.0 / 7.0 / 8.3 (7.5, 10.9), four of 64 6.6 / 6.6 / 7.5 (6.8, 12.9), 16 of 5 6.6 / 6.4 / 7.4 (6.5, 11.5)
+// What such a call still pays, about 1 us, is workgroups that look the batch up and leave.
+inline void planSplit(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq, Plan &plan) {
     const long long seqs = in.num_seqs > 0 ? static_cast<long long>(in.num_seqs) : 1;
     const long long kv_heads = static_cast<long long>(in.num_kv_heads);
     const long long blocks = seqs * ((rows_per_seq + 63) / 64) * kv_heads;
     const long long tokens = static_cast<long long>(in.max_num_blocks_per_seq) * static_cast<long long>(in.page_block_size);
     const long long slots = static_cast<long long>(dev.compute_units) * (in.head_size <= 192 ? 2 : 1);
+    plan.max_parts = 1;
     if (blocks <= 0) {
-        return 1;
+        return;
     }
-    const long long most = std::min(std::min(slots / blocks, (tokens + kSplitTableTokens - 1) / kSplitTableTokens),
-                                    static_cast<long long>(kMaxSplitParts));
-    const double us_per_1000 = in.head_size == 64 ? 11 : in.head_size == 128 ? 14 : in.head_size == 192 ? 22
-                             : in.head_size == 256 ? 20 : 41;
-    const double walk = us_per_1000 * 1e-3 * static_cast<double>(tokens);
+    const int most = static_cast<int>(std::min(std::min(slots / blocks, (tokens + kSplitTableTokens - 1) / kSplitTableTokens),
+                                               static_cast<long long>(kMaxSplitParts)));
+    const double us_per_token = 1e-3 * (in.head_size == 64 ? 11 : in.head_size == 128 ? 14 : in.head_size == 192 ? 22
+                                      : in.head_size == 256 ? 20 : 41);
     const double row_bytes = static_cast<double>(rows_per_seq) * seqs * kv_heads * in.value_size * sizeof(float);
-    const double row_cost = 0.9e-6 * row_bytes, merge_cost = 3.0;
-    int best = 1;
-    double least = 0.8 * walk;
-    for (int p = 2; p <= most; ++p) {
-        const double shared = blocks * p > dev.compute_units && in.head_size <= 192 ? 1.4 : 1.0;
-        const double t = shared * walk / p + row_cost * p + merge_cost;
-        if (t < least) {
-            best = p, least = t;
+    const double meet_cost = 3.5, part_cost = 0.3e-6 * row_bytes;
+    // time of the best split of a walk of `t` tokens
+    auto split = [&](double t, int &best) {
+        double least = 1e30;
+        for (int p = 2; p <= most && (p - 1) * kSplitTableTokens < t; ++p) {
+            const double shared = blocks * p > dev.compute_units && in.head_size <= 192 ? 1.4 : 1.0;
+            const double us = shared * us_per_token * t / p + meet_cost + part_cost * p;
+            if (us < least) {
+                best = p, least = us;
+            }
         }
+        return least;
+    };
+    int best = 1, any = 1;
+    if (split(static_cast<double>(tokens), best) >= 0.8 * us_per_token * static_cast<double>(tokens)) {
+        return;
     }
-    return best;
+    plan.max_parts = best;
+    long long from = kSplitTableTokens;
+    while (from < tokens && split(static_cast<double>(from), any) >= us_per_token * static_cast<double>(from)) {
+        from += 64;
+    }
+    plan.split_from = static_cast<int>(from);
+    plan.part_cost = static_cast<float>(part_cost / us_per_token);
 }
 
 inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev) {
@@ -153,11 +176,16 @@ inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::Dev
     plan.compute_units = dev.compute_units;
     // (a forced number of rows asks for those kernels as they are)
     const bool rows_forced = std::getenv("INFINIOP_AMD_PREFILL_GROUPS") != nullptr;
-    plan.max_parts = plan.tiled && r == 1 && !rows_forced ? splitParts(in, dev, rows_per_seq) : 1;
+    plan.max_parts = 1;
+    if (plan.tiled && r == 1 && !rows_forced) {
+        planSplit(in, dev, rows_per_seq, plan);
+    }
     if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_PARTS")) {
         const int forced = std::atoi(env);
         if (plan.tiled && r == 1 && forced >= 1 && forced <= kMaxSplitParts) {
             plan.max_parts = forced;
+            plan.split_from = 0;
+            plan.part_cost = 0.0f;
         }
     }
     if (plan.max_parts > 1) {
@@ -165,8 +193,15 @@ inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::Dev
         if (part_rows >= (size_t{1} << 31)) { // a knob's doing: more workgroups than a launch has
             plan.max_parts = 1;
         }
+        // Workgroups that merge a block, up to eight (two rows per wavefront), while all of them are one and a half rounds of
+        // the device: us with 1 / 2 / 4 / 8 at 64 blocks (one sequence of 100 tokens over 1 900, eight parts)
+        // 33.7 / 24.7 / 19.9 / 17.4, at 160 (four of 64, four parts) 41.1 / 31.3 / 26.8 / 28.7
+        const long long grid = (rows / 64 + seqs) * static_cast<long long>(in.num_kv_heads);
+        const long long room = 3 * dev.compute_units * (in.head_size <= 192 ? 2 : 1) / 2 / grid;
+        plan.merge_workgroups = room >= 8 ? 8 : (room >= 4 ? 4 : (room >= 2 ? 2 : 1));
         plan.part_acc_bytes = part_rows * in.value_size * sizeof(float);
         plan.part_ml_bytes = part_rows * 2 * sizeof(float);
+        plan.part_flags_bytes = part_rows * sizeof(unsigned long long);
     }
     const size_t widest = in.head_size > in.value_size ? in.head_size : in.value_size;
     plan.dims_per_lane = static_cast<int>((widest + 63) / 64);

@@ -40,6 +40,7 @@
 
 #include "../../paged_attention/amd/decode_tiled.h"
 #include "prefill_common.h"
+#include "prefill_split.h"
 
 namespace op::paged_attention_prefill::amd {
 
@@ -91,9 +92,11 @@ constexpr unsigned kLongestFirstRounds = 6; // of workgroups that the device hol
 // workgroup beyond the last block.
 // `span` receives the sequence's span as the lane that looked at it read it (lane reads: loading it again
 // would be one more memory round trip at the head of every workgroup).
-template <typename Tindex>
+// With ASK, `place` is asked for x once the batch is known: the number of row blocks and whether any sequence holds tokens
+// enough to be split (of more than 64 sequences, only that there are too many to know); below 0 is none.
+template <typename Tindex, bool ASK = false, typename Place = int>
 __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int block_rows, int x, int &seq, int &block,
-                                             SeqSpan &span_out) {
+                                             SeqSpan &span_out, Place place = {}) {
     const int block_tokens = max(block_rows / a.group, 1);
     for (int base = 0; base < a.num_seqs; base += 64) {
         const int idx = base + lane;
@@ -107,6 +110,15 @@ __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int
         }
         const int incl = waveInclusiveSum(nb);
         const int blocks = __builtin_amdgcn_readlane(incl, 63);
+        if constexpr (ASK) {
+            if (base == 0) {
+                const bool all = a.num_seqs <= 64;
+                x = place(all ? blocks : 0x7fffffff, !all || __builtin_amdgcn_ballot_w64(nb > 0 && span.kv_len >= a.split_from) != 0);
+                if (x < 0) {
+                    return false;
+                }
+            }
+        }
         if (x >= blocks) {
             x -= blocks;
             continue;
@@ -184,21 +196,8 @@ constexpr int prefillStepTokens() { return (KHEAD <= 128 || KHEAD == 256 || (KHE
 template <int KHEAD, int R>
 constexpr int prefillWorkgroupsPerUnit() { return (KHEAD <= 128 || (KHEAD == 192 && R == 1)) ? 2 : 1; }
 
-// The steps of one row block as its parts take them (SPLIT below): `per` each, `used` parts in all, at most max_parts and
-// none shorter than kSplitTokens but the last.
-constexpr int kSplitTokens = 128;
-struct SplitSteps {
-    int per, used;
-};
-__device__ __forceinline__ SplitSteps splitSteps(int n_steps, int step_tokens, int max_parts) {
-    const int parts = min(max_parts, (n_steps * step_tokens + kSplitTokens - 1) / kSplitTokens);
-    SplitSteps s;
-    s.per = (n_steps + parts - 1) / parts;
-    s.used = (n_steps + s.per - 1) / s.per;
-    return s;
-}
-
-// SPLIT: a.max_parts workgroups per row block, each for a range of its steps (prefill_split.h).
+// SPLIT: up to a.max_parts workgroups per row block, each for a range of its steps, and behind all of those
+// a.merge_workgroups that merge the parts of a block (prefill_split.h).
 // PLAIN: no ALiBi and scale > 0. The running maximum is then kept in units of the raw dot product
 // (a positive scale keeps the order) and each probability costs one fused multiply-add and one exp2.
 template <typename T, typename Tindex, int KHEAD, int VHEAD, int R, bool PLAIN, bool SPLIT = false>
@@ -229,14 +228,37 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     // KV head fastest: workgroup ids go round-robin over the 8 accelerator dies, so with 8 (or a
     // multiple of 8) KV heads every die works on its own heads and the row blocks resident on a die
     // at one time are neighbours that stream the same K/V through that die's L2.
-    const int kv_head = blockIdx.x % a.num_kv_heads;
-    const int part = SPLIT ? static_cast<int>(blockIdx.x / a.num_kv_heads) % a.max_parts : 0;
-    const int block_index = SPLIT ? blockIdx.x / a.num_kv_heads / a.max_parts : blockIdx.x / a.num_kv_heads;
+    // SPLIT: the parts of a block are next to one another in the grid, so that the workgroups of one part of several blocks of
+    // a sequence, which read the same keys and values, come at the same distance: few dies have them. Where the lengths show
+    // that every block stays whole, blocks are numbered as without SPLIT (a workgroup in max_parts would have work, and some
+    // compute units two of those, others none), and the rest of the grid leaves.
+    int kv_head = blockIdx.x % a.num_kv_heads;
+    int block_index = blockIdx.x / a.num_kv_heads;
+    int part = 0; // of the block, or which of those that merge it
+    const bool merges = SPLIT && blockIdx.x >= a.part_workgroups;
+    auto place = [&](int blocks, bool any_split) {
+        if (any_split) {
+            const unsigned at = merges ? blockIdx.x - a.part_workgroups : blockIdx.x;
+            const unsigned per_block = merges ? a.merge_workgroups : a.max_parts;
+            kv_head = at % a.num_kv_heads;
+            block_index = at / a.num_kv_heads / per_block;
+            part = at / a.num_kv_heads - block_index * per_block;
+        } else if (merges) {
+            return -1;
+        }
+        return block_index < min(blocks, a.row_blocks) ? block_index : -1;
+    };
 
     int seq = 0, block = 0;
     SeqSpan span;
-    if (!findRowBlock<Tindex>(a, lane, BM, block_index, seq, block, span)) {
-        return;
+    if constexpr (SPLIT) {
+        if (!findRowBlock<Tindex, true>(a, lane, BM, 0, seq, block, span, place)) {
+            return;
+        }
+    } else {
+        if (!findRowBlock<Tindex>(a, lane, BM, block_index, seq, block, span)) {
+            return;
+        }
     }
     const int total_rows = span.q_len * a.group; // > 0 here
     const int block_row0 = block * BM;
@@ -252,13 +274,19 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     int first_step = 0, n_steps = all_steps; // this workgroup's: [first_step, n_steps)
     bool partial = false;                    // ... are not all of them
     if constexpr (SPLIT) {
-        const SplitSteps split = splitSteps(all_steps, BN, a.max_parts);
+        const SplitSteps split = splitSteps(a, block_visible, all_steps);
+        if (merges) {
+            if (split.used > 1) {
+                mergeParts<T, VHEAD>(a, span, block_index, kv_head, block_row0, last_row, 4 * part + w, 4 * a.merge_workgroups, split, BN, lane);
+            }
+            return;
+        }
+        if (part >= split.used) {
+            return;
+        }
         first_step = part * split.per;
         n_steps = min(first_step + split.per, all_steps);
         partial = split.used > 1;
-        if (first_step >= all_steps) {
-            return;
-        }
     }
 
     // ---- this lane's columns: row c of each of the wavefront's R column groups ----
@@ -695,29 +723,9 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     }
 
     if constexpr (SPLIT) {
-        if (partial) { // the state as it is; rows that see nothing of these steps leave m = -inf and zeros
-            const int64_t row0 = ((static_cast<int64_t>(block_index) * a.num_kv_heads + kv_head) * a.max_parts + part) * BM + 16 * w;
-            float *acc = a.part_acc + row0 * VHEAD;
-            const int rows = last_row + 1 - block_row0 - 16 * w; // of this wavefront's 16 that exist (or more, or none)
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                if (4 * g + rr < rows) {
-#pragma unroll
-                    for (int e = 0; e < G::kColsV; ++e) {
-                        acc[(4 * g + rr) * VHEAD + 16 * e + c] = o[0][e][rr];
-                    }
-                }
-            }
-            float *ml = reinterpret_cast<float *>(a.part_ml + row0);
-            if (g == 0) {
-                ml[2 * c] = m[0] * unit;
-            }
-            if (c == 0) {
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) {
-                    ml[2 * (4 * g + rr) + 1] = ol[0][rr];
-                }
-            }
+        if (partial) { // the state as it is; rows that see nothing of these steps leave m = -inf
+            publishPart<VHEAD>(a, partFirstRow(a, block_index, kv_head, part) + 16 * w, o[0], ol[0], m[0] * unit,
+                               partRowExists(block_row0 + 16 * w + c, last_row, visible[0]), lane);
             return;
         }
     }

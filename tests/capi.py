@@ -89,6 +89,12 @@ def create_paged_attention_prefill(handle, out, q, k_cache, v_cache, block_table
     return status, op
 
 
+def workspace_size_prefill(op) -> int:
+    size = c_size_t(123)
+    L.check_error(L.LIBINFINIOP.infiniopGetPagedAttentionPrefillWorkspaceSize(op, ctypes.byref(size)))
+    return size.value
+
+
 def run_paged_attention_prefill(handle, q, k_cache, v_cache, block_tables, seq_lens, cum_seq_lens_q, scale, alibi=None,
                                 out=None, stream=None):
     """Full create / query / run / destroy cycle on device tensors (the sequence of calls of

@@ -10,9 +10,10 @@ import numpy as np
 import pytest
 import torch
 
+from infinicore_amd import libinfiniop as L
 from infinicore_amd import workloads
 
-from capi import run_paged_attention_prefill
+from capi import create_paged_attention_prefill, run_paged_attention_prefill, workspace_size_prefill
 from test_paged_attention_gpu import DEV, ORACLE_THREADS, assert_close, climbing_keys
 
 pytestmark = pytest.mark.gpu
@@ -386,6 +387,104 @@ def test_parts_that_a_row_sees_nothing_of_add_nothing(gpu_handle, oracle, monkey
     assert_close(got, want[rows], "split_inf", want_f32[rows])
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_weights_of_zero_count_as_in_a_whole_block(gpu_handle, monkeypatch, value):
+    """Tokens that a row sees, in a part whose weight underflows: 0 times what is not finite is NaN, split or not."""
+    cfg = prefill_config("split_zero", torch.float16, 1, 4, 2, 128, 16, (5, 5), (600, 600), seed=4)
+    inp = workloads.make_prefill_inputs(cfg)
+    inp.q.fill_(4.0)
+    inp.k_cache.fill_(4.0)
+    for t in range(128):  # scores 2 ^ -500 below the others'
+        inp.k_cache[int(inp.block_tables[0, t // 16]), :, t % 16] = -4.0
+    inp.v_cache[int(inp.block_tables[0, 0]), 0, 3] = value
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    got = []
+    for parts in ("1", "5"):  # of 128 tokens each
+        monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", parts)
+        got.append(run_paged_attention_prefill(gpu_handle, *dev, inp.scale).cpu())
+    for out in got:
+        assert torch.isnan(out[:, :2]).all() and torch.isfinite(out[:, 2:]).all()
+
+
+def test_split_of_more_sequences_than_lanes(gpu_handle, oracle, monkeypatch):
+    """Two rounds of the block search in parts and merge; whole and split blocks, sequences without new tokens."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", "3")
+    cfg = prefill_config("split_many", torch.bfloat16, 70, 4, 2, 64, 16, (1, 40), (0, 500), seed=70)
+    inp = workloads.make_prefill_inputs(cfg)
+    new = (inp.cum_seq_lens_q[1:] - inp.cum_seq_lens_q[:-1]).clone()
+    new[5::9] = 0
+    inp.cum_seq_lens_q[1:] = torch.cumsum(new, 0)
+    inp.q = inp.q[:int(inp.cum_seq_lens_q[-1])].clone()
+    run_case(gpu_handle, oracle, inp)
+
+
+@pytest.mark.parametrize("D,H,Hkv", [(64, 10, 2), (128, 32, 8), (256, 14, 2), (576, 16, 1)])
+@pytest.mark.parametrize("new,history", [((1, 5), (0, 0)), ((1, 150), (0, 0)), ((1, 30), (0, 1500))])
+def test_plans_for_tables_wider_than_the_sequences(gpu_handle, oracle, D, H, Hkv, new, history):
+    """The plan splits for what the table can hold, the kernel by what the sequences hold: none, some or all blocks."""
+    cfg = workloads.PrefillConfig(f"wide{D}", torch.bfloat16, 3, H, Hkv, D, 16, *new, *history, seed=D,
+                                  value_size=512 if D == 576 else D)
+    inp = workloads.make_prefill_inputs(cfg)
+    rng = np.random.default_rng(D)
+    wide = torch.from_numpy(rng.integers(-5, inp.k_cache.shape[0] + 5, (3, 2048)))  # entries nobody may follow
+    wide[:, :inp.block_tables.shape[1]] = inp.block_tables
+    inp.block_tables = wide
+    q, k, v = (t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache))
+    status, op = create_paged_attention_prefill(gpu_handle, torch.empty(*q.shape[:2], v.shape[-1], dtype=q.dtype, device=DEV), q, k, v,
+                                                wide.to(DEV), inp.seq_lens.to(DEV), inp.cum_seq_lens_q.to(DEV), None, inp.scale)
+    assert status == 0 and workspace_size_prefill(op) > 0
+    assert L.LIBINFINIOP.infiniopDestroyPagedAttentionPrefillDescriptor(op) == 0
+    run_case(gpu_handle, oracle, inp)
+
+
+@pytest.mark.parametrize("D,H,Hkv", [(64, 16, 16), (128, 32, 8), (192, 32, 8), (256, 28, 4), (576, 16, 1)])
+def test_lengths_round_the_one_a_split_pays_from(gpu_handle, oracle, D, H, Hkv):
+    """One sequence on a wide table, its length round every multiple of a step up to well past that point: below it no block
+    of the batch is split, from it on some are, whatever the rounding to steps."""
+    lens = [64 * n + d for n in range(2, 11) for d in (-33, -1, 0, 1)]
+    cfg = workloads.PrefillConfig(f"threshold{D}", torch.bfloat16, 1, H, Hkv, D, 16, 3, 3, 700, 700, seed=D,
+                                  value_size=512 if D == 576 else D)
+    inp = workloads.make_prefill_inputs(cfg)
+    inp.block_tables = torch.nn.functional.pad(inp.block_tables, (0, 1000))
+    for n in lens:
+        inp.seq_lens = torch.tensor([n])
+        run_case(gpu_handle, oracle, inp, what=f"threshold{D} {n}")
+
+
+def test_replays_with_other_lengths(gpu_handle, oracle):
+    """A captured call whose lengths change in place between replays: more parts, fewer, none, and again. The tokens that
+    parts leave in the workspace are the captured call's in every replay."""
+    from infinicore_amd import ops
+
+    cfg = prefill_config("replays", torch.bfloat16, 2, 32, 8, 128, 16, (6, 6), (4000, 4000), seed=5)
+    inp = workloads.make_prefill_inputs(cfg)
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    cases = []
+    for lens, new in (((4006, 4006), (6, 6)), ((700, 3), (6, 6)), ((4006, 1500), (1, 11)), ((9, 6), (6, 6)), ((130, 2600), (12, 0)),
+                      ((4006, 4006), (6, 6))):
+        inp.seq_lens = torch.tensor(lens)
+        inp.cum_seq_lens_q = torch.tensor([0, new[0], new[0] + new[1]])
+        want = oracle.paged_attention_prefill(inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q,
+                                              inp.scale, num_threads=ORACLE_THREADS, return_fp32=True,
+                                              out=torch.full(inp.q.shape, SENTINEL, dtype=cfg.dtype))
+        cases.append((inp.seq_lens.to(DEV), inp.cum_seq_lens_q.to(DEV), want))
+    out = torch.empty_like(dev[0])
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        ops.paged_attention_prefill(*dev, None, inp.scale, out=out)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            ops.paged_attention_prefill(*dev, None, inp.scale, out=out)
+    for _ in range(2):
+        for lens, cum, want in cases:
+            dev[4].copy_(lens), dev[5].copy_(cum), out.fill_(SENTINEL)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_close(out.cpu(), want[0], f"lengths {lens.tolist()}", want[1])
+
+
 def test_split_call_without_its_workspace_and_under_capture(gpu_handle, oracle):
     """The plan's own split: the same result without the workspace (unsplit), and from a replayed graph."""
     from infinicore_amd import ops
@@ -451,21 +550,54 @@ def test_scores_that_climb_along_the_sequence(gpu_handle, oracle, monkeypatch, g
     inp.q[:] = (inp.q.float() * scale_rows).to(cfg.dtype)
     run_case(gpu_handle, oracle, inp)
 
+
+def row_block_grid(inp, rows):
+    """Workgroups of a launch with `rows` rows per workgroup, and how many the device holds at a time."""
+    cfg = inp.config
+    resident = 2 if inp.q.shape[2] <= 128 else 1
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    grid = (inp.q.shape[0] * cfg.num_heads // cfg.num_kv_heads // rows + cfg.num_seqs) * cfg.num_kv_heads
+    return grid, resident * units
+
+
 @pytest.mark.parametrize("groups", ["1", "2"])
-@pytest.mark.parametrize("seqs,heads,kv_heads", [(1, 8, 2), (1, 96, 96), (7, 10, 2), (9, 32, 32), (64, 4, 1), (65, 12, 4), (130, 4, 2)])
+@pytest.mark.parametrize("seqs,heads,kv_heads", [(1, 288, 288), (7, 50, 10), (9, 64, 64), (64, 16, 8), (65, 36, 12), (130, 16, 8)])
 def test_every_row_block_of_a_ragged_batch_is_worked_on(gpu_handle, oracle, monkeypatch, groups, seqs, heads, kv_heads):
-    """Blocks are dealt longest first where there are more than 512 workgroups: equal lengths, sequences without new tokens, single tokens, totals below the new
-    tokens, a group that does not divide the rows of a workgroup, more sequences than lanes."""
+    """Blocks are dealt longest first from one to six rounds of workgroups: equal lengths, sequences without new tokens, single
+    tokens, totals below the new tokens, a group that does not divide the rows of a workgroup, more sequences than lanes."""
     monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
     cfg = prefill_config("order", torch.float16, seqs, heads, kv_heads, 64, 16, (1, 90 if seqs > 8 else 400), (0, 300), seed=seqs)
-    inp = workloads.make_prefill_inputs(cfg)
+    inp = ragged(workloads.make_prefill_inputs(cfg))
+    grid, slots = row_block_grid(inp, 64 * int(groups))
+    assert slots < grid <= 6 * slots, (grid, slots)
+    run_case(gpu_handle, oracle, inp)
+
+
+def ragged(inp):
     new = (inp.cum_seq_lens_q[1:] - inp.cum_seq_lens_q[:-1]).clone()
-    if seqs > 1:
+    if new.shape[0] > 1:
         new[1] = 0
         new[2::7] = 1
         inp.seq_lens[3::5] = int(inp.seq_lens.min())  # equal lengths, some below the number of new tokens
     inp.cum_seq_lens_q[1:] = torch.cumsum(new, 0)
     inp.q = inp.q[:int(inp.cum_seq_lens_q[-1])].clone()
+    return inp
+
+
+@pytest.mark.parametrize("groups", ["1", "2"])
+def test_every_row_block_of_a_ragged_latent_batch_is_worked_on(gpu_handle, oracle, monkeypatch, groups):
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
+    inp = ragged(mla_inputs("latent_order", torch.bfloat16, 30, 16, 16, (1, 200), (0, 100), seed=12))
+    grid, slots = row_block_grid(inp, 64 * int(groups))
+    assert slots < grid <= 6 * slots, (grid, slots)
+    run_case(gpu_handle, oracle, inp)
+
+
+def test_plain_block_order_beyond_six_rounds(gpu_handle, oracle):
+    cfg = prefill_config("plain_order", torch.float16, 65, 64, 64, 64, 16, (1, 90), (0, 100), seed=6)
+    inp = ragged(workloads.make_prefill_inputs(cfg))
+    grid, slots = row_block_grid(inp, 64)
+    assert grid > 6 * slots
     run_case(gpu_handle, oracle, inp)
 
 
