@@ -5,6 +5,10 @@
 // (src/infiniop/ops/paged_attention/cuda/kernel_v2.cuh:134-336) on a 64-lane wavefront. It does
 // not share K/V between the query heads of a group and is only used for shapes the tiled kernel
 // does not cover.
+// WAVES > 1: one workgroup per (query head, sequence), whose wavefronts share the sequence's tokens and merge through
+// LDS. For calls on a plan of one partition per sequence, made for the tiled kernel, whose operands turn out not to
+// be 16-byte aligned: there is no workspace for partial results, and one wavefront per sequence and head took up to
+// @GEN@.
 #ifndef INFINICORE_AMD_PA_DECODE_GENERIC_H
 #define INFINICORE_AMD_PA_DECODE_GENERIC_H
 
@@ -12,13 +16,14 @@
 
 namespace op::paged_attention::amd {
 
-template <typename T, typename Tindex, int DIMS_PER_LANE>
-__global__ void __launch_bounds__(64) decodeGenericKernel(DecodeArgs a) {
+template <typename T, typename Tindex, int DIMS_PER_LANE, int WAVES = 1>
+__global__ void __launch_bounds__(64 * WAVES) decodeGenericKernel(DecodeArgs a) {
     using S = typename T::storage;
     const int part = blockIdx.x;
     const int head = blockIdx.y;
     const int seq = blockIdx.z;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = WAVES > 1 ? static_cast<int>(threadIdx.x >> 6) : 0;
 
     const int64_t len64 = loadIndex<Tindex>(a.seq_lens, seq);
     if (len64 <= 0) {
@@ -26,11 +31,12 @@ __global__ void __launch_bounds__(64) decodeGenericKernel(DecodeArgs a) {
     }
     const int64_t max_len = static_cast<int64_t>(a.max_blocks_per_seq) * a.block_size;
     const int len = static_cast<int>(len64 < max_len ? len64 : max_len);
-    const int start = part * a.partition_tokens;
-    if (start >= len) {
+    const int tokens = WAVES > 1 ? (len + WAVES - 1) / WAVES : a.partition_tokens;
+    const int start = (WAVES > 1 ? wave : part) * tokens;
+    if (WAVES == 1 && start >= len) {
         return;
     }
-    const int end = min(len, start + a.partition_tokens);
+    const int end = min(len, start + tokens);
     const int kv_head = head / a.group;
     const float slope = a.alibi_slopes ? a.alibi_slopes[head] : 0.0f;
 
@@ -87,7 +93,43 @@ __global__ void __launch_bounds__(64) decodeGenericKernel(DecodeArgs a) {
         }
     }
 
-    if (len <= a.partition_tokens) {
+    if constexpr (WAVES > 1) { // (a wavefront without tokens has m = -inf, l = 0 and zeros)
+        __shared__ float other_m[WAVES], other_l[WAVES], other_acc[WAVES][DIMS_PER_LANE * 64];
+#pragma unroll
+        for (int i = 0; i < DIMS_PER_LANE; ++i) {
+            other_acc[wave][lane + 64 * i] = acc[i];
+        }
+        if (lane == 0) {
+            other_m[wave] = m;
+            other_l[wave] = l;
+        }
+        __syncthreads();
+        if (wave != 0) {
+            return;
+        }
+        const float m_own = m;
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) {
+            m = fmaxf(m, other_m[w]);
+        }
+        const float own = m_own == -INFINITY ? 0.0f : fastExp2(m_own - m);
+        l *= own;
+#pragma unroll
+        for (int i = 0; i < DIMS_PER_LANE; ++i) {
+            acc[i] *= own;
+        }
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) {
+            const float f = other_m[w] == -INFINITY ? 0.0f : fastExp2(other_m[w] - m);
+            l += other_l[w] * f;
+#pragma unroll
+            for (int i = 0; i < DIMS_PER_LANE; ++i) {
+                acc[i] += other_acc[w][lane + 64 * i] * f;
+            }
+        }
+    }
+
+    if (WAVES > 1 || len <= a.partition_tokens) {
         // whole sequence in this partition: normalise and store (kernel_v2.cuh:318-335)
         const float inv_l = 1.0f / (l + 1e-6f);
         S *o_ptr = static_cast<S *>(a.out) + seq * a.o_stride + head * a.o_head_stride;

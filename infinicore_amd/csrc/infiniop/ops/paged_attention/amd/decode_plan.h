@@ -34,6 +34,7 @@ struct Plan {
     int latent_chunks;     // that kernel: 16-head chunks that share a workgroup: 1 (eight wavefronts for the one chunk), 4 or 8 (a wavefront each)
     bool latent_roles;     // four chunks: a wavefront for the scores and a wavefront for the values of each (decodeMlaRolesKernel)
     bool partition_forced; // INFINIOP_AMD_PA_PARTITION set: the 64-head kernel keeps exactly that size
+    bool one_partition;    // grid schedule, tiled: every sequence is one partition (short tables)
     int partition_tokens;  // grid schedule: tokens per unit of work
     int max_partitions;    // grid schedule: partitions the longest representable sequence needs
     // A descriptor planned for the work-equalising schedule runs the element-wise kernel when the operands of
@@ -113,25 +114,36 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
                         && static_cast<long long>(in.num_seqs) * stream_count * max_tiles <= 64LL * dev.compute_units;
     // Short sequences, one partition each: nothing to merge, so no second launch and no partial rows. A wavefront then walks
     // its sequence from end to end (4.6 us and 0.024 / 0.035 / 0.045 / 0.056 us per token at head 64 / 128 / 192 / 256, alone
-    // on its SIMD); any cut costs two launches (10 us) and the time its bytes take. One partition where its walk is a tenth
-    // shorter than that, for the tokens the table can hold; up to 1 024 tokens were measured. us per call, cut as before /
-    // one partition (bf16, 32 / 8 heads, lengths from an eighth of the table up):
-    //   * head 128: 48 sequences of up to 96 11.1 / 7.2, 192 13.0 / 10.7, 512 (stays cut) 19.3 / 22.2; 128 of up to 192
-    //     20.1 / 14.5, 512 34.3 / 32.2; 256 of up to 96 24.4 / 14.7, 320 42.5 / 38.6
-    //   * head 64: 256 of up to 192 22.9 / 15.7; 128 of up to 768 28.6 / 27.1, 1 008 34.0 / 34.3 (of 806 - 1 008 46.5 / 41.5)
-    //   * head 256 with 28 / 4 heads: 128 of up to 192 24.1 / 16.4, 512 44.6 / 36.3; 48 of up to 192 (stays cut) 13.8 / 15.3
+    // on its SIMD). What a cut call takes is two launches and the time its bytes take, but the lengths are not known
+    // here, and a batch in which one sequence is as long as the table and the others are short is over much sooner than a full
+    // one: in 9.4 us and 1.88 us per 1 000 units when cut, and in the walk of that one sequence when not. So: where the walk
+    // over the whole table is the shorter one for such a batch too. us per call, one partition / the better of the cut
+    // schedules, for one full and the others 16 tokens, every eighth full and the others an eighth, all full (bf16, 32 / 8 heads):
+    //   * head 128: 24 sequences of up to 128 8.1 / 9.5, 8.2 / 9.9, 8.2 / 10.1; 128 of up to 192 10.5 / 11.4, 11.3 / 12.9, 12.9 /
+    //     18.6; 256 of up to 192 11.8 / 13.9, 17.0 / 18.9, 27.8 / 35.5; stay cut: 24 of up to 192 10.0 / 9.6, 10.2 / 9.8, 10.4 / 10.5;
+    //     128 of up to 512 22.4 / 12.8, 24.5 / 17.4; 256 of up to 1 024 42 / 16, 83 / 47
+    //   * head 64: 48 of up to 192 9.0 / 9.5, 9.2 / 9.4, 9.4 / 11.1; 256 of up to 288 13.1 / 13.2, 15.8 / 18.6, 22.1 / 29.4; stay
+    //     cut: 24 of up to 288 11.0 / 9.1, 11.2 / 9.4, 11.2 / 10.4; 128 of up to 512 17.6 / 12.6, 18.9 / 15.7
+    //   * head 192: 128 of up to 144 11.0 / 12.1, 12.0 / 14.7, 15.2 / 22.3; stay cut: 256 of up to 192 14.9 / 15.1, 26.0 / 22.7
+    //   * head 256, 28 / 4 heads: 256 of up to 112 11.5 / 16.4, 15.4 / 19.0, 19.7 / 25.4; stay cut: 128 of up to 160 13.2 / 11.8
     const double unit_tokens = static_cast<double>(units) * static_cast<double>(max_tokens);
     const double head_cols = static_cast<double>(in.head_size);
-    // (a forced schedule asks for its cuts)
-    const bool one_partition = plan.tiled && !latent_head && std::getenv("INFINIOP_AMD_PA_SCHEDULE") == nullptr
-                            && max_tokens <= 1024 && max_tokens <= kPageIdsPerWave * bs
-                            && 4.6 + (0.0135 + 1.65e-4 * head_cols) * max_tokens < 0.9 * (10.0 + 4e-7 * head_cols * unit_tokens);
-    // From 67 MB of keys and values on (two wavefronts per SIMD in partitions of 64 tokens at head 128), small jobs are cut
-    // into 128 tokens instead of 64: half the partial rows and workgroup starts. us with 64 / 128: 32 / 8 heads of 128, 2
-    // sequences of up to 8 192 21.2 / 17.7, 8 of 500 - 2 048 15.4 / 13.9, 48 of 409 - 512 26.1 / 23.4; 28 / 4 heads of 256, 2 of
-    // up to 8 192 23.2 / 18.7, 48 of 806 - 1 008 49.7 / 47.0. Below it the walk is what counts: 16 of up to 768 with heads of
-    // 64 11.0 / 12.2, with 28 / 4 heads of 256 14.2 / 16.4.
-    const bool long_partitions = small_job && head_cols * unit_tokens >= 131072.0 * 128.0;
+    const double walk = 4.6 + (0.0135 + 1.65e-4 * head_cols) * static_cast<double>(max_tokens);
+    // (a forced schedule, size or merge asks for its cuts)
+    const bool cut_forced = std::getenv("INFINIOP_AMD_PA_SCHEDULE") != nullptr || std::getenv("INFINIOP_AMD_PA_PARTITION") != nullptr
+                         || std::getenv("INFINIOP_AMD_PA_MERGE") != nullptr;
+    plan.one_partition = plan.tiled && !latent_head && !cut_forced && max_tokens > 0 && max_tokens <= kPageIdsPerWave * bs
+                      && walk < 9.4 + 1.88e-3 * static_cast<double>(units < 2048 ? units : 2048)
+                      && walk < 0.9 * (10.0 + 4e-7 * head_cols * unit_tokens);
+    // From 67 MB of keys and values on (two wavefronts per SIMD in partitions of 64 tokens at head 128), few long sequences are
+    // cut into 128 tokens instead of 64: half the partial rows and workgroup starts. us with 64 / 128, lengths of 300, of 1 000,
+    // the whole table, and one whole among others of 50:
+    //   * 32 / 8 heads of 128: 2 sequences of up to 8 192 12.0 / 11.9, 12.8 / 11.9, 19.5 / 15.8, 15.6 / 12.5; 4 of up to 4 096 12.3 /
+    //     11.5, 13.2 / 12.4, 18.1 / 15.1, 11.2 / 11.4; stay at 64: 8 of up to 2 048 10.3 / 11.3, 13.5 / 12.2, 17.1 / 14.5, 10.0 / 11.0
+    //   * 16 heads of 64, 4 of up to 4 096: 12.3 / 10.2, 12.8 / 12.5, 18.3 / 15.5, 11.2 / 10.7; 192: 14.2 / 12.9, 15.0 / 13.8, 23.1 /
+    //     20.2, 12.5 / 12.9
+    //   * stay at 64: 28 / 4 heads of 256, 4 of up to 4 096 12.8 / 14.3, 13.4 / 14.7, 19.9 / 17.1, 12.2 / 14.6
+    const bool long_partitions = small_job && in.head_size <= 192 && max_tokens >= 4096 && head_cols * unit_tokens >= 131072.0 * 128.0;
     // A unit of the latent-attention kernel leaves 32 KiB of partial results and advances one tile per
     // ~2 us however many units there are: fewer, longer units measured best there (more units end the
     // decode kernel sooner, but writing and merging their partial results costs more than that gains).
@@ -182,7 +194,7 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
     if (long_partitions && p < 128) {
         p = 128;
     }
-    if (one_partition && max_tokens > 0) {
+    if (plan.one_partition) {
         p = max_tokens;
     }
     if (const char *env = std::getenv("INFINIOP_AMD_PA_PARTITION")) {
@@ -225,7 +237,7 @@ inline Plan makePlan(const PagedAttentionInfo &in, const device::amd::DeviceInfo
     // arithmetic below divides by both counts)
     const bool can_balance = plan.tiled && !latent_head && flat_axis_fits && in.num_seqs <= static_cast<size_t>(kBalancedMaxSeqs)
                           && in.num_seqs > 0 && stream_count > 0;
-    plan.balanced = can_balance && !small_job && !one_partition;
+    plan.balanced = can_balance && !small_job && !plan.one_partition;
     if (const char *env = std::getenv("INFINIOP_AMD_PA_SCHEDULE")) {
         if (std::strcmp(env, "grid") == 0) {
             plan.balanced = false;

@@ -25,6 +25,15 @@ namespace {
 template <typename T, typename Tindex>
 void launchGeneric(const DecodeArgs &a, const Plan &plan, hipStream_t stream) {
     const dim3 grid(a.max_partitions, a.num_heads, a.num_seqs);
+    if (plan.one_partition && a.partition_tokens > 64) { // heads of 64 .. 256 that the tiled kernel cannot take now
+        switch (plan.dims_per_lane) {
+        case 1: decodeGenericKernel<T, Tindex, 1, 4><<<grid, 256, 0, stream>>>(a); break;
+        case 2: decodeGenericKernel<T, Tindex, 2, 4><<<grid, 256, 0, stream>>>(a); break;
+        case 3: decodeGenericKernel<T, Tindex, 3, 4><<<grid, 256, 0, stream>>>(a); break;
+        default: decodeGenericKernel<T, Tindex, 4, 4><<<grid, 256, 0, stream>>>(a); break;
+        }
+        return;
+    }
     switch (plan.dims_per_lane) {
     case 1: decodeGenericKernel<T, Tindex, 1><<<grid, 64, 0, stream>>>(a); break;
     case 2: decodeGenericKernel<T, Tindex, 2><<<grid, 64, 0, stream>>>(a); break;

@@ -9,10 +9,10 @@ import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
 KNOBS = ("INFINIOP_AMD_PA_KERNEL", "INFINIOP_AMD_PA_SCHEDULE", "INFINIOP_AMD_PA_LATENT_KERNEL", "INFINIOP_AMD_PA_LATENT_HEADS",
-         "INFINIOP_AMD_PA_PARTITION", "INFINIOP_AMD_PA_WAVES_PER_CU")
+         "INFINIOP_AMD_PA_PARTITION", "INFINIOP_AMD_PA_WAVES_PER_CU", "INFINIOP_AMD_PA_MERGE")
 FIELDS = ("tiled", "balanced", "latent_wide", "partition_tokens", "max_partitions", "fallback_partition_tokens",
           "fallback_max_partitions", "waves_per_stream", "workspace_bytes", "launchable", "acc_bytes", "ml_bytes",
-          "latent_chunks", "latent_roles")
+          "latent_chunks", "latent_roles", "one_partition")
 
 
 def build_probe(directory):
@@ -166,3 +166,32 @@ def test_head_chunks_that_share_a_latent_attention_workgroup(probe, monkeypatch)
     assert chunks(200, 128) == (1, 4)
     monkeypatch.setenv("INFINIOP_AMD_PA_LATENT_HEADS", "96")
     assert chunks(200, 128) == (1, 8)       # not a size the kernels have: ignored
+
+
+@pytest.mark.parametrize("head,heads,kv,seqs,table,one", [
+    (128, 32, 8, 24, 128, True), (128, 32, 8, 128, 192, True), (128, 32, 8, 256, 192, True), (128, 32, 8, 24, 192, False),
+    (128, 32, 8, 128, 512, False), (128, 32, 8, 256, 1024, False), (64, 32, 8, 48, 192, True), (64, 32, 8, 256, 288, True),
+    (64, 32, 8, 24, 288, False), (64, 16, 16, 256, 512, False), (192, 32, 8, 128, 144, True), (192, 32, 8, 256, 192, False),
+    (256, 28, 4, 256, 112, True), (256, 28, 4, 128, 160, False)])
+def test_short_sequences_are_one_partition_where_one_long_one_is_no_loss(probe, monkeypatch, head, heads, kv, seqs, table, one):
+    pl = probe(seqs, heads, kv, head, 16, table // 16)
+    assert pl["one_partition"] == one
+    if one:
+        assert pl["max_partitions"] == 1 and pl["partition_tokens"] == table and pl["workspace_bytes"] == 0
+        assert not pl["balanced"] and pl["fallback_max_partitions"] == 1
+        for knob, value in (("SCHEDULE", "balanced"), ("PARTITION", "64"), ("MERGE", "kernel")):
+            monkeypatch.setenv("INFINIOP_AMD_PA_" + knob, value)
+            forced = probe(seqs, heads, kv, head, 16, table // 16)
+            assert not forced["one_partition"] and forced["workspace_bytes"] > 0
+            monkeypatch.delenv("INFINIOP_AMD_PA_" + knob)
+    else:
+        assert pl["workspace_bytes"] > 0
+
+
+@pytest.mark.parametrize("head,heads,kv,seqs,table,tokens", [
+    (128, 32, 8, 2, 8192, 128), (128, 32, 8, 4, 4096, 128), (64, 16, 16, 4, 4096, 128), (192, 32, 8, 4, 4096, 128),
+    (128, 32, 8, 8, 2048, 64), (64, 16, 16, 8, 1024, 64), (256, 28, 4, 4, 4096, 64), (256, 28, 4, 2, 8192, 64),
+    (128, 32, 8, 1, 4096, 64)])
+def test_few_long_sequences_have_longer_partitions(probe, head, heads, kv, seqs, table, tokens):
+    pl = probe(seqs, heads, kv, head, 16, table // 16)
+    assert not pl["balanced"] and pl["partition_tokens"] == tokens

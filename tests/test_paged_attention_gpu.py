@@ -208,8 +208,8 @@ def test_tiled_kernels_other_head_sizes(gpu_handle, oracle, monkeypatch, D, dtyp
     run_case(gpu_handle, oracle, inp)
 
 
-@pytest.mark.parametrize("D,H,Hkv,bs,table", [(64, 16, 16, 16, 1024), (64, 40, 2, 32, 96), (128, 8, 2, 16, 512),
-                                                (128, 5, 1, 128, 128), (192, 16, 2, 16, 320), (256, 14, 2, 64, 192)])
+@pytest.mark.parametrize("D,H,Hkv,bs,table", [(64, 16, 16, 16, 256), (64, 40, 2, 32, 96), (128, 8, 2, 16, 128),
+                                                (128, 5, 1, 128, 128), (192, 16, 2, 16, 96), (256, 14, 2, 16, 80)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_short_sequences_in_one_partition(gpu_handle, oracle, monkeypatch, dtype, D, H, Hkv, bs, table):
     """The default plan of many short sequences: a partition as long as the table holds, no workspace; lengths round its
@@ -234,6 +234,45 @@ def test_short_sequences_in_one_partition(gpu_handle, oracle, monkeypatch, dtype
     got = run_paged_attention(gpu_handle, q, k, v, bt, sl, inp.scale, alibi=slopes.to(DEV))
     want, want_f32 = oracle_of(oracle, inp, alibi_slopes=slopes, return_fp32=True)
     assert_close(got[1:], want[1:], cfg.name, want_f32[1:])
+
+
+@pytest.mark.parametrize("D,H,Hkv,table", [(64, 4, 2, 128), (128, 32, 8, 128), (192, 8, 2, 96), (256, 14, 2, 80)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_unaligned_operands_of_a_one_partition_plan(gpu_handle, oracle, monkeypatch, dtype, D, H, Hkv, table):
+    """The element-wise kernel shares a sequence between the wavefronts of a workgroup: lengths that leave some of them
+    without tokens, slopes, and values that are not finite in a share whose weight is nothing."""
+    monkeypatch.delenv("INFINIOP_AMD_PA_SCHEDULE", raising=False)
+    B = max(48, 4096 // Hkv // 8)
+    cfg = custom(f"unaligned_one_{D}", dtype, B, H, Hkv, D, 16, 0, 40, seed=D, spare_block_fraction=0.1)
+    inp = workloads.make_decode_inputs(cfg)
+    rng = np.random.default_rng(D)
+    inp.block_tables = torch.from_numpy(rng.integers(0, inp.k_cache.shape[0], (B, table // 16))).to(torch.int64)
+    inp.seq_lens = torch.from_numpy(rng.integers(1, table + 1, B)).to(torch.int64)
+    edges = [0, 1, 2, 3, 4, 5, 7, 63, 64, 65, table - 1, table]
+    inp.seq_lens[:len(edges)] = torch.tensor(edges)
+    q, k, v, bt, sl = to_device(inp)
+
+    def shifted(t):
+        room = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)[1:]
+        return room.copy_(t.flatten()).view(t.shape)
+
+    k, v = shifted(k), shifted(v)
+    status, op = create_paged_attention(gpu_handle, torch.empty_like(q), q, k, v, bt, sl, None, inp.scale)
+    assert status == 0 and workspace_size_attention(op) == 0
+    assert L.LIBINFINIOP.infiniopDestroyPagedAttentionDescriptor(op) == 0
+    for slopes in (None, torch.tensor([2.0 ** -(i % 6 + 1) for i in range(H)])):
+        got = run_paged_attention(gpu_handle, q, k, v, bt, sl, inp.scale, alibi=None if slopes is None else slopes.to(DEV))
+        want, want_f32 = oracle_of(oracle, inp, alibi_slopes=slopes, return_fp32=True)
+        assert_close(got[1:], want[1:], cfg.name, want_f32[1:])
+    # the last share of a sequence scores 2 ^ -500 below the others and holds an infinity
+    inp.block_tables[:] = torch.arange(table // 16) % inp.k_cache.shape[0]
+    q.fill_(4.0), k.fill_(4.0)
+    k[table // 16 - 1, :, 15] = -64.0
+    v[table // 16 - 1, 0, 15] = float("inf")
+    full = torch.full_like(sl, table)
+    got = run_paged_attention(gpu_handle, q, k, v, inp.block_tables.to(DEV), full, inp.scale).cpu()
+    group = H // Hkv
+    assert not torch.isfinite(got[:, :group]).any() and torch.isfinite(got[:, group:]).all()
 
 
 @pytest.mark.parametrize("D", [64, 192, 256])
