@@ -21,7 +21,7 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     jobs = jobs or min(8, os.cpu_count() or 1)
     if force:
         subprocess.run(["make", "-C", str(CSRC_DIR), "clean"], check=True, capture_output=not verbose)
-    proc = subprocess.run(["make", "-C", str(CSRC_DIR), f"-j{jobs}", f"PYTHON={sys.executable}"], capture_output=not verbose, text=True)
+    proc = subprocess.run(["make", "-C", str(CSRC_DIR), f"-j{jobs}", f"PYTHON={sys.executable}", "all", "torch"], capture_output=not verbose, text=True)
     if proc.returncode != 0:
         raise RuntimeError("building the InfiniOP AMD libraries failed:\n" + (proc.stdout or "") + (proc.stderr or ""))
     if not libraries_present():

@@ -40,10 +40,13 @@ _handles: dict[int, object] = {}
 
 
 def _load_native():
-    """csrc/torch_ops: from the package's own library folder, whichever build of the C libraries is in use."""
-    path = Path(__file__).resolve().parent / "lib" / "_torch_ops.so"
-    if not path.is_file():
-        raise ImportError(f"{path} not found: build it first (python -m infinicore_amd.build, or __graft_entry__.build())")
+    """csrc/torch_ops: built beside the C libraries in use, or else the one in the package's own library folder (a build of
+    the C libraries alone; the extension gets their functions below, so any will do)."""
+    folders = (lib.LIB_DIR, Path(__file__).resolve().parent / "lib")
+    path = next((f / "_torch_ops.so" for f in folders if (f / "_torch_ops.so").is_file()), None)
+    if path is None:
+        raise ImportError(f"_torch_ops.so not found in {folders[0]}: build it first (python -m infinicore_amd.build, "
+                          "__graft_entry__.build(), or make -C infinicore_amd/csrc torch)")
     spec = importlib.util.spec_from_file_location("infinicore_amd._torch_ops", path)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)

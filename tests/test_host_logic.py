@@ -107,3 +107,24 @@ def test_prefill_flops_count_visible_pairs():
     assert new.tolist() == [3, 3] and history.tolist() == [10, 10]
     pairs = 2 * (11 + 12 + 13)
     assert workloads.prefill_flops(cfg, new, history) == pairs * 4 * 4 * 128
+
+
+def test_the_c_libraries_build_without_torch():
+    """`make` alone: nothing of the Python extension, whatever Python is or is not there."""
+    proc = subprocess.run(["make", "-n", "-B", "-C", str(ROOT / "infinicore_amd" / "csrc"), "PYTHON=/no/such/python"],
+                          capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and "libinfinicore_ops.so" in proc.stdout and "torch" not in proc.stdout
+
+
+@pytest.mark.parametrize("beside", [False, True])
+def test_the_extension_of_another_build_of_the_libraries(tmp_path, beside):
+    """INFINICORE_AMD_LIB_DIR with and without a _torch_ops.so of its own: infinicore_amd.ops can be imported either way."""
+    import os
+
+    built = ROOT / "infinicore_amd" / "lib"
+    for name in ("libinfinirt.so", "libinfiniop.so", "libinfinicore_ops.so", *(["_torch_ops.so"] if beside else [])):
+        (tmp_path / name).symlink_to(built / name)
+    proc = subprocess.run([sys.executable, "-c", "from infinicore_amd import ops; print(ops._native.__file__)"], text=True,
+                          capture_output=True, timeout=300, cwd=ROOT, env={**os.environ, "INFINICORE_AMD_LIB_DIR": str(tmp_path)})
+    assert proc.returncode == 0, proc.stderr
+    assert Path(proc.stdout.strip()).parent == (tmp_path if beside else built)
