@@ -24,6 +24,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -219,12 +220,13 @@ PyObject *call(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     const c10::DeviceIndex device = on.device().index();
     at::Tensor allocated;
     if (op.has_out && t[0] == nullptr) {
-        if (on.dim() == 0 || t[3]->dim() == 0) {
-            PyErr_SetString(PyExc_IndexError, "q and v_cache have no dimensions");
+        if (t[3]->dim() == 0) {
+            PyErr_SetString(PyExc_IndexError, "v_cache has no dimensions");
             return nullptr;
         }
-        c10::DimVector shape(on.sizes().begin(), on.sizes().end());
-        shape.back() = t[3]->size(-1);
+        // (a query without dimensions is refused by the operator, with its status)
+        c10::DimVector shape(on.sizes().begin(), on.sizes().begin() + std::max<int64_t>(on.dim() - 1, 0));
+        shape.push_back(t[3]->size(-1));
         allocated = at::empty(shape, at::TensorOptions().dtype(on.scalar_type()).device(on.device()));
         t[0] = &allocated;
     }

@@ -45,6 +45,16 @@ def test_operators_refuse_host_tensors():
         ops.paged_attention(t, t, t, t, t)
 
 
+def test_a_query_without_dimensions_is_refused_by_the_operator():
+    from infinicore_amd import ops
+
+    kc = torch.zeros(4, 2, 16, 64, dtype=torch.float16, device=DEV)
+    bt, sl = torch.zeros(1, 2, dtype=torch.int64, device=DEV), torch.ones(1, dtype=torch.int64, device=DEV)
+    with pytest.raises(RuntimeError) as refused:
+        ops.paged_attention(torch.zeros((), dtype=torch.float16, device=DEV), kc, kc, bt, sl)
+    assert hasattr(refused.value, "status")
+
+
 def test_plans_by_metadata_stream_and_thread(oracle):
     """More shapes than the cache keeps, called again after their plans went; strided queries of one shape; several
     threads on streams of their own at once."""
