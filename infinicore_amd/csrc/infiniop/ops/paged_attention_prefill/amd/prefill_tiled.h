@@ -77,7 +77,18 @@ __device__ __forceinline__ uint4 loadLane16Cached(const char *uniform_base, uint
 // Rows of one workgroup for R column groups per wavefront.
 __host__ __device__ constexpr int prefillBlockRows(int r) { return 64 * r; }
 
-constexpr unsigned kLongestFirstRounds = 6; // of workgroups that the device holds at a time
+// Row blocks are dealt longest first (findRowBlock) where the grid is between these many rounds of the workgroups that the
+// device holds at a time, else as the sequences come. Measured, bf16, mean over random orders of a batch, as they come ->
+// longest first: head 128 at 1.0 - 1.2 rounds 0.87 - 1.05 of the time (100.7 -> 89.3 us, 80.9 -> 83.6), 1.5 - 2.3 mostly 0.8 -
+// 0.95 (119.2 -> 98.3), 3.0 201 -> 189.5, 5.2 344.7 -> 336.3, 6.8 113.6 -> 116.2 and 448.7 -> 444.9, 10 782 -> 807, 12 837 ->
+// 866. Latent heads at 1.1 266.8 -> 222, 2.8 480 -> 442, 5 809 -> 773, 6.5 1 038 -> 1 013, 24 1 457 -> 1 473. Head 64 loses up
+// to 1.7 rounds in 14 shapes of 16 (1.03: 50.4 -> 53.9, 1.14: 59.7 -> 63.6, 1.7: 16.6 -> 17.8) and gains from there (1.8: 83.3
+// -> 76.1, 2.9: 127 -> 111, 5.4: 256.5 -> 247.5), 9.5 455 -> 479. Within one round the
+// order makes no difference; why it loses just above one and far beyond six was not measured.
+template <int KHEAD>
+constexpr bool longestFirst(unsigned long long grid, unsigned long long slots) {
+    return (KHEAD == 64 ? 4 * grid > 7 * slots : grid > slots) && grid <= 6 * slots;
+}
 
 // Which (sequence, row block) workgroup `x` of a KV head works on: the x-th longest block of the batch. The dispatcher
 // starts workgroups in the order of their numbers, so the long blocks of a ragged batch start first and the last round
@@ -141,7 +152,7 @@ __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int
         // blocks of this lane's sequence with a key of at least `key`
         auto countFrom = [&](int key) { return min(max(top - key + 1, 0), nb); };
         auto blocksFrom = [&](int key) { return __builtin_amdgcn_readlane(waveInclusiveSum(countFrom(key)), 63); };
-        // the largest key with more than x blocks from it on: at least that of the x + 1 longest blocks of one sequence
+        // lo ends as the largest key with more than x blocks from it on; every block has at least the first lo, none hi
         int lo = __builtin_amdgcn_readfirstlane(-waveMaxInt(nb > 0 ? nb - 1 - top : -0x40000000));
         int hi = __builtin_amdgcn_readfirstlane(waveMaxInt(nb > 0 ? top : -0x40000000)) + 1;
         while (hi - lo > 1) { // blocksFrom(lo) > x >= blocksFrom(hi)

@@ -566,7 +566,7 @@ def test_every_row_block_of_a_ragged_batch_is_worked_on(gpu_handle, oracle, monk
     """Blocks are dealt longest first from one to six rounds of workgroups: equal lengths, sequences without new tokens, single
     tokens, totals below the new tokens, a group that does not divide the rows of a workgroup, more sequences than lanes."""
     monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", groups)
-    cfg = prefill_config("order", torch.float16, seqs, heads, kv_heads, 64, 16, (1, 90 if seqs > 8 else 400), (0, 300), seed=seqs)
+    cfg = prefill_config("order", torch.float16, seqs, heads, kv_heads, 128, 16, (1, 90 if seqs > 8 else 400), (0, 300), seed=seqs)
     inp = ragged(workloads.make_prefill_inputs(cfg))
     grid, slots = row_block_grid(inp, 64 * int(groups))
     assert slots < grid <= 6 * slots, (grid, slots)
@@ -593,11 +593,14 @@ def test_every_row_block_of_a_ragged_latent_batch_is_worked_on(gpu_handle, oracl
     run_case(gpu_handle, oracle, inp)
 
 
-def test_plain_block_order_beyond_six_rounds(gpu_handle, oracle):
-    cfg = prefill_config("plain_order", torch.float16, 65, 64, 64, 64, 16, (1, 90), (0, 100), seed=6)
+@pytest.mark.parametrize("heads,rounds", [(40, (6, 12)), (20, (1.75, 6)), (7, (1, 1.75))])
+def test_block_order_of_head_64(gpu_handle, oracle, monkeypatch, heads, rounds):
+    """Longest first between seven quarters and six rounds of workgroups, as the sequences come on either side."""
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_GROUPS", "1")
+    cfg = prefill_config("plain_order", torch.float16, 65, heads, heads, 64, 16, (1, 90), (0, 100), seed=6)
     inp = ragged(workloads.make_prefill_inputs(cfg))
     grid, slots = row_block_grid(inp, 64)
-    assert grid > 6 * slots
+    assert rounds[0] * slots < grid <= rounds[1] * slots, (grid, slots)
     run_case(gpu_handle, oracle, inp)
 
 
