@@ -7,8 +7,8 @@
 // does not cover.
 // WAVES > 1: one workgroup per (query head, sequence), whose wavefronts share the sequence's tokens and merge through
 // LDS. For calls on a plan of one partition per sequence, made for the tiled kernel, whose operands turn out not to
-// be 16-byte aligned: there is no workspace for partial results, and one wavefront per sequence and head took up to
-// @GEN@.
+// be 16-byte aligned: there is no workspace for partial results. 48 sequences of up to 96 tokens, 32 / 8 heads of 128: one
+// wavefront per sequence and head 132 us, four 41, cut into partitions of 64 tokens with the merge kernel 102.
 #ifndef INFINICORE_AMD_PA_DECODE_GENERIC_H
 #define INFINICORE_AMD_PA_DECODE_GENERIC_H
 

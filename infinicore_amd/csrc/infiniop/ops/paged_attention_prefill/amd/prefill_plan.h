@@ -31,20 +31,23 @@ inline bool multipleOf8(ptrdiff_t x) { return (x % 8) == 0; }
 
 // Latent attention (keys of 576): 64 or 128 rows per workgroup, as 1 or 2. One workgroup per compute unit with either
 // kernel, and one of 128 rows (prefill_latent.h) takes 1.4 x as long as one of 64 over the same tokens. So 128 rows where
-// they save more than a third of the rounds of workgroups. Measured, us with 64 rows / with 128, by 64-row blocks (16
-// heads, bf16, 256 compute units):
-//   * three rounds against two: 640 blocks over 2 000 tokens of history 312 / 320, 740 330 / 340; 64 sequences of 40
-//     without history 41 / 43
-//   * four against two: 1 000 over 2 000 452 / 385, over 500 212 / 197; 16 sequences of 200 without history 57 / 56, four
-//     of 900 113.5 / 114.5; five against three: 100 sequences of 50 75 / 70
+// they save more than a third of the rounds of workgroups. Measured with the longest blocks first (prefill_tiled.h), us with
+// 64 rows / with 128, by 64-row blocks (16 heads, bf16, 256 compute units):
+//   * three rounds against two: 640 blocks over 2 000 tokens of history 317 / 295, 740 303 / 292; 64 sequences of 40
+//     without history 36 / 37; 16 of 60 - 260 without history 44.6 / 43.4, over 500 - 4 000 311 / 268; six of 200 - 750 over up
+//     to 3 000 234 / 206. The line was drawn where blocks started as the sequences come (312 / 320 and 330 / 340 then); in this
+//     order 128 rows would be the better ones for most of these
+//   * four against two: 1 000 over 2 000 409 / 310, over 500 150 / 119; 16 sequences of 200 without history 58 / 48, four
+//     of 900 114 / 90, 16 of 100 - 380 over 500 - 4 000 435 / 350; five against three: 100 sequences of 50 75 / 63, 40 of 30 -
+//     190 over up to 3 000 357 / 291
 //   * two rounds against one: the second round is short where a block's tokens grow along the sequence (the longest blocks
 //     start first, the last ones fit behind the shortest of the first round) or where sequences differ in length, and
-//     then 128 rows only make the longest block longer. One sequence without history, 275 blocks 64 / 90, 500 111 / 142; two
-//     of 900 60 / 74; four of 128 - 512 over 1 024 - 8 192 419 / 501. With much history and equal lengths it is a whole
-//     round: four of 500 over 2 000 219 / 176. The lengths of several sequences are not known here: 64 rows. For one
+//     then 128 rows only make the longest block longer. One sequence without history, 275 blocks 60 / 85, 500 112 / 141; two
+//     of 900 59 / 72; four of 128 - 512 over 1 024 - 8 192 423 / 502. With much history and equal lengths it is a whole
+//     round: four of 500 over 2 000 221 / 178. The lengths of several sequences are not known here: 64 rows. For one
 //     sequence the table says how much history there can be, and its blocks are dealt in order: block 256 + j starts when
 //     block 256 - j ends, after 2 history + 2 n (1 - 256 / blocks) tokens of n new ones in all, against 1.4 (history + n).
-//     1 600 over 1 200: 177 / 189, over 3 000 327 / 299; 2 000 over 1 000 194 / 205, over 2 000 276 / 267. (A table wider
+//     1 600 over 1 200: 180 / 191, over 3 000 334 / 300; 2 000 over 1 000 199 / 202, over 2 000 283 / 265. (A table wider
 //     than the sequence looks like history.)
 inline int latentRowGroups(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq) {
     const long long units = dev.compute_units > 0 ? dev.compute_units : 1;

@@ -50,18 +50,23 @@ def no_knobs(monkeypatch):
 
 
 def makespan(new, hist, group, block_rows, units=256):
-    """Time of the batch in tokens of a 64-row block: workgroups start in grid order (last sequence first, within it the
-    blocks that see most first), each on the compute unit that is free first. A block of 128 rows takes 1.4 x as long as
-    one of 64 over the same tokens; the start of a block is worth some 40 tokens."""
-    free = [0.0] * units
-    end = 0.0
+    """Time of the batch in tokens of a 64-row block: workgroups start in grid order, each on the compute unit that is free
+    first. The grid has the longest blocks first where it is one to six rounds of workgroups, else the last sequence first and
+    within it the blocks that see most. A block of 128 rows takes 1.4 x as long as one of 64 over the same tokens; the start
+    of a block is worth some 40 tokens."""
+    blocks = []
     for n, h in reversed(list(zip(new, hist))):
         rows = n * group
-        for b in reversed(range(-(-rows // block_rows))):
-            sees = h + (min((b + 1) * block_rows, rows) - 1) // group + 1
-            t = heapq.heappop(free) + (40 + sees) * (1.4 if block_rows == 128 else 1.0)
-            end = max(end, t)
-            heapq.heappush(free, t)
+        blocks += [h + (min((b + 1) * block_rows, rows) - 1) // group + 1 for b in reversed(range(-(-rows // block_rows)))]
+    grid = sum(new) * group // block_rows + len(new)
+    if units < grid <= 6 * units:
+        blocks.sort(reverse=True)
+    free = [0.0] * units
+    end = 0.0
+    for sees in blocks:
+        t = heapq.heappop(free) + (40 + sees) * (1.4 if block_rows == 128 else 1.0)
+        end = max(end, t)
+        heapq.heappush(free, t)
     return end
 
 
