@@ -201,13 +201,16 @@ infiniStatus_t Descriptor::calculate(void *workspace, size_t workspace_size, voi
     // the element-wise kernel instead.
     a.max_parts = 1;
     if (plan.max_parts > 1 && workspace != nullptr && workspace_size >= _workspace_size) {
+        const size_t left_marks = static_cast<size_t>(plan.row_block_grid) * kMergeWavefronts; // behind the tokens
         char *ws = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~static_cast<uintptr_t>(255));
         a.part_acc = reinterpret_cast<float *>(ws);
         a.part_ml = reinterpret_cast<float2 *>(ws + plan.part_acc_bytes);
         a.part_flags = reinterpret_cast<unsigned long long *>(ws + plan.part_acc_bytes + plan.part_ml_bytes);
+        a.part_left = a.part_flags + (plan.part_flags_bytes / sizeof(unsigned long long) - left_marks);
         a.token = device::amd::nextToken();
         a.max_parts = plan.max_parts;
         a.merge_workgroups = plan.merge_workgroups;
+        a.merge_polls = plan.merge_polls;
         a.split_from = plan.split_from;
         a.part_cost = plan.part_cost;
     } // without the workspace it asks for, the call runs unsplit

@@ -48,12 +48,14 @@ struct PrefillArgs {
     float *part_acc;                // [row block][KV head][part][64 rows][value_size]
     float2 *part_ml;                // [row block][KV head][part][64 rows] reference point (log2), denominator
     unsigned long long *part_flags; // [row block][KV head][part][64 rows] `token` once the row is there
+    unsigned long long *part_left;  // [row block][KV head][32 merging wavefronts] `token` where one has left rows to the parts
     unsigned long long token;       // of this call
     int32_t row_blocks;             // an upper bound of the row blocks: the grid holds that many
     unsigned part_workgroups;       // row_blocks x KV heads x max_parts; the workgroups that merge come behind
     int32_t max_parts;
     int32_t merge_workgroups; // of a row block and KV head: 1, 2, 4 or 8
     int32_t split_from; // tokens that a row block sees, at least, to be split
+    int32_t merge_polls; // that a merging wavefront waits for a row's parts
     float part_cost;    // what the rows of one more part cost, in tokens of a workgroup's walk
 };
 

@@ -20,6 +20,8 @@ struct Plan {
     int compute_units;
     int max_parts;       // tiled, 64 rows: workgroups that may share a row block (prefill_split.h); 1 = none is split
     int merge_workgroups; // of a row block: 1, 2, 4 or 8
+    long long row_block_grid; // row blocks x KV heads that the batch can have
+    int merge_polls;     // of a wavefront that merges, before it leaves its rows to the parts (prefill_split.h)
     int split_from;      // tokens from which a row block is split, and what a further part costs in tokens (PrefillArgs)
     float part_cost;
     size_t part_acc_bytes, part_ml_bytes, part_flags_bytes; // workspace of the parts, each a multiple of 256 bytes
@@ -64,6 +66,10 @@ inline int latentRowGroups(const PagedAttentionPrefillInfo &in, const device::am
     return 2 * rounds64 > 3 * rounds128 ? 2 : 1;
 }
 
+constexpr int kMergeWavefronts = 32; // that merge a block, at most: eight workgroups of four
+// ~1 us each, 2 ms in all: far beyond the time between the parts of a call that has the device for itself (a walk of
+// 16 384 tokens in two parts takes 0.1 ms, latent 0.35)
+constexpr int kMergePolls = 2000;
 constexpr int kMaxSplitParts = 64; // the merge forms the weights of a row with a lane per part
 constexpr long long kSplitTableTokens = 128; // a part per that many tokens at most (kSplitTokens of prefill_split.h)
 
@@ -204,7 +210,12 @@ inline Plan makePlan(const PagedAttentionPrefillInfo &in, const device::amd::Dev
         plan.merge_workgroups = room >= 8 ? 8 : (room >= 4 ? 4 : (room >= 2 ? 2 : 1));
         plan.part_acc_bytes = part_rows * in.value_size * sizeof(float);
         plan.part_ml_bytes = part_rows * 2 * sizeof(float);
-        plan.part_flags_bytes = part_rows * sizeof(unsigned long long);
+        plan.row_block_grid = grid;
+        plan.part_flags_bytes = (part_rows + static_cast<size_t>(grid) * kMergeWavefronts) * sizeof(unsigned long long);
+        plan.merge_polls = kMergePolls;
+        if (const char *env = std::getenv("INFINIOP_AMD_PREFILL_MERGE_POLLS")) {
+            plan.merge_polls = std::max(0, std::atoi(env));
+        }
     }
     const size_t widest = in.head_size > in.value_size ? in.head_size : in.value_size;
     plan.dims_per_lane = static_cast<int>((widest + 63) / 64);

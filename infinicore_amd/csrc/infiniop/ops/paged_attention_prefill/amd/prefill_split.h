@@ -15,20 +15,26 @@
 // Parts and merge meet as pieces and reader of the decode kernel do (decode_common.h has the accesses): a part's wavefront
 // writes its rows through to memory, waits for that, and stores the call's token beside each row; the wavefront that merges
 // a row polls the tokens of its parts, reads past the caches, and clears the tokens, so that a replay of the call starts
-// clean. Every row that a part flags is merged by exactly one wavefront, and only flagged rows are waited for: both sides
-// go by partRowExists. Merging workgroups come last in the grid and parts wait for nobody, so with in-order dispatch they
-// always end; a wait is bounded all the same.
+// clean. Every row that a part flags is merged, and only flagged rows are waited for: both sides
+// go by partRowExists.
+// Merging workgroups come last in the grid and parts wait for nobody, so alone on the device they always get their rows. Beside
+// another such call, on another stream, they may not: each die takes the workgroups of its queues in its own order, and
+// merging workgroups of one call can hold the places that the other's parts need on one die, and the other way round on another.
+// So a merging wavefront waits for merge_polls at most. Then it marks its rows as left (part_left), looks once more, and
+// goes; a part's wavefront looks for such marks after its tokens are in memory, and merges the rows that are complete. Whichever
+// of the two came second sees the other's word, so every row is merged: by either, or by both from the same rows to the same
+// bits. Nothing waits without bound and no row depends on who waited.
 #ifndef INFINICORE_AMD_PA_PREFILL_SPLIT_H
 #define INFINICORE_AMD_PA_PREFILL_SPLIT_H
 
 #include "../../paged_attention/amd/decode_reduce.h"
 #include "prefill_common.h"
+#include "prefill_plan.h"
 
 namespace op::paged_attention_prefill::amd {
 
 constexpr int kPartRows = 64;       // rows of a split block
 constexpr int kSplitTokens = 128;   // a block has a part per that many tokens, at most
-constexpr int kMergeSpinLimit = 1 << 22; // polls (~0.5 us each) before a wait gives up
 
 // The steps of one row block as its parts take them: `per` each, `used` parts in all.
 struct SplitSteps {
@@ -118,10 +124,15 @@ __device__ __forceinline__ float mergeSum(float x) {
     return laneOf(x, 63);
 }
 
-// One wavefront merges its rows of a split block: wave, wave + waves, .. of all that exist, two at a time. A part's row is
+__device__ __forceinline__ unsigned long long *leftMarks(const PrefillArgs &a, int block_index, int kv_head) {
+    return a.part_left + (static_cast<int64_t>(block_index) * a.num_kv_heads + kv_head) * kMergeWavefronts;
+}
+
+// One wavefront merges its rows of a split block: wave, wave + waves, .. of all that exist, two at a time. With WAITS it is
+// that wavefront of the merging workgroups; else a part's in its place, which takes the rows that are complete. A part's row is
 // VHEAD / 4 chunks of 16 bytes; up to head 128 several parts' rows fit the lanes of one load. The code is kept short: it
 // runs once or a few times per launch, out of a cold instruction cache (all rows of a wavefront unrolled: twice as long).
-template <typename T, int VHEAD>
+template <typename T, int VHEAD, bool WAITS>
 __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &span, int block_index, int kv_head, int block_row0,
                                            int last_row, int wave, int waves, SplitSteps split, int step_tokens, int lane) {
     using namespace op::paged_attention::amd;
@@ -138,6 +149,11 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
     const int side = kSide > 1 ? lane / kChunks : 0;
     const int chunk = kSide > 1 ? lane % kChunks : lane;
     const int part_tokens = split.per * step_tokens;
+    unsigned long long *const mark = leftMarks(a, block_index, kv_head) + wave;
+    bool left = !WAITS; // the rows may be merged by somebody else as well
+    if (WAITS && lane == 0) {
+        storeAgent(mark, 0); // (a replay that left rows)
+    }
 
     for (int first_row = wave; first_row < kPartRows; first_row += N * waves) {
         int token[N], head[N], seen[N]; // seen: parts that the row sees any token of
@@ -155,8 +171,8 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
         if (!any) {
             return; // nor any row behind
         }
-        bool arrived = true;
-        for (int spins = 0;; ++spins) {
+        bool complete = false;
+        for (int polls = 0;; ++polls) {
             bool here = true;
 #pragma unroll
             for (int n = 0; n < N; ++n) {
@@ -164,18 +180,24 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
                     here = here && loadAgent(flags + kPartRows * lane + first_row + n * waves) == a.token;
                 }
             }
-            if (__builtin_amdgcn_ballot_w64(!here) == 0) {
+            complete = __builtin_amdgcn_ballot_w64(!here) == 0;
+            if (complete || left) {
                 break;
             }
-            if (spins > kMergeSpinLimit) {
-                arrived = false; // not with in-order dispatch; never wait for ever
-                break;
+            if (polls >= a.merge_polls) {
+                left = true;
+                if (lane == 0) {
+                    storeAgent(mark, a.token);
+                }
+                waitVectorMemory(); // the mark is in memory before the last look
+            } else {
+                __builtin_amdgcn_s_sleep(1);
             }
-            __builtin_amdgcn_s_sleep(1);
+        }
+        if (!complete) {
+            continue; // the part that completes them finds the mark; or somebody has merged them
         }
         compilerMemoryBarrier(); // the loads below stay below the flag loads above
-        // (a wait that ran out must not pass for a result: NaN)
-        const float one = arrived ? 1.0f : __builtin_nanf("");
         float2 ml[N];
         float4 sum[N][kMine];
 #pragma unroll
@@ -246,7 +268,7 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
             if (!exists[n]) {
                 continue;
             }
-            const float inv_l = one / (l[n] + 1e-6f);
+            const float inv_l = 1.0f / (l[n] + 1e-6f);
             unsigned short *o_ptr = reinterpret_cast<unsigned short *>(static_cast<S *>(a.out) + (span.q_start + token[n]) * a.o_stride + head[n] * a.o_head_stride);
 #pragma unroll
             for (int k = 0; k < kMine; ++k) {
@@ -263,6 +285,21 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
                 storeAgent(flags + kPartRows * lane + first_row + n * waves, 0);
             }
         }
+    }
+}
+
+// A part's wavefront, its rows published: the rows that merging wavefronts of this block have left.
+template <typename T, int VHEAD>
+__device__ __forceinline__ void mergeLeftRows(const PrefillArgs &a, const SeqSpan &span, int block_index, int kv_head, int block_row0,
+                                              int last_row, SplitSteps split, int step_tokens, int lane) {
+    using namespace op::paged_attention::amd;
+    const int waves = 4 * a.merge_workgroups;
+    waitVectorMemory(); // this wavefront's tokens are in memory before it looks for marks
+    unsigned long long marked = __builtin_amdgcn_ballot_w64(lane < waves && loadAgent(leftMarks(a, block_index, kv_head) + lane) == a.token);
+    while (marked != 0) {
+        const int wave = __builtin_ctzll(marked);
+        marked &= marked - 1;
+        mergeParts<T, VHEAD, false>(a, span, block_index, kv_head, block_row0, last_row, wave, waves, split, step_tokens, lane);
     }
 }
 

@@ -284,11 +284,12 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     const int all_steps = (block_visible + BN - 1) / BN;
     int first_step = 0, n_steps = all_steps; // this workgroup's: [first_step, n_steps)
     bool partial = false;                    // ... are not all of them
+    SplitSteps split{0, 1};
     if constexpr (SPLIT) {
-        const SplitSteps split = splitSteps(a, block_visible, all_steps);
+        split = splitSteps(a, block_visible, all_steps);
         if (merges) {
             if (split.used > 1) {
-                mergeParts<T, VHEAD>(a, span, block_index, kv_head, block_row0, last_row, 4 * part + w, 4 * a.merge_workgroups, split, BN, lane);
+                mergeParts<T, VHEAD, true>(a, span, block_index, kv_head, block_row0, last_row, 4 * part + w, 4 * a.merge_workgroups, split, BN, lane);
             }
             return;
         }
@@ -737,6 +738,7 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         if (partial) { // the state as it is; rows that see nothing of these steps leave m = -inf
             publishPart<VHEAD>(a, partFirstRow(a, block_index, kv_head, part) + 16 * w, o[0], ol[0], m[0] * unit,
                                partRowExists(block_row0 + 16 * w + c, last_row, visible[0]), lane);
+            mergeLeftRows<T, VHEAD>(a, span, block_index, kv_head, block_row0, last_row, split, BN, lane);
             return;
         }
     }

@@ -339,6 +339,7 @@ def test_head_576_column_layout_garbage_alibi_and_int32(gpu_handle, oracle):
     slopes = torch.tensor([2.0 ** -(i % 5 + 1) for i in range(8)], dtype=torch.float32)
     run_case(gpu_handle, oracle, inp, alibi=slopes, index_dtype=torch.int32)
 
+
 # ---- row blocks whose tokens several workgroups share ----------------------------------------------------------
 
 @pytest.mark.parametrize("parts", ["2", "5", "64"])
@@ -360,6 +361,36 @@ def test_split_row_blocks(gpu_handle, oracle, monkeypatch, D, H, Hkv, bs, dtype,
     inp.seq_lens = torch.tensor(lens, dtype=torch.int64)
     run_case(gpu_handle, oracle, inp, index_dtype=idx)
     run_case(gpu_handle, oracle, inp, alibi=torch.tensor([2.0 ** -(i % 5 + 1) for i in range(H)]), index_dtype=idx)
+
+
+@pytest.mark.parametrize("polls", ["0", "3"])
+@pytest.mark.parametrize("D,H,Hkv,new,history,parts", [
+    (64, 10, 2, (1, 40), (300, 1300), "5"), (128, 32, 8, (60, 70), (2000, 2100), "4"), (192, 6, 6, (1, 150), (100, 900), "7"),
+    (256, 14, 2, (1, 20), (1, 3000), "64"), (576, 16, 1, (1, 9), (100, 900), "6")])
+def test_rows_that_a_merging_wavefront_leaves_are_merged_by_the_parts(gpu_handle, monkeypatch, D, H, Hkv, new, history, parts, polls):
+    """Next to no patience: most rows are left to the part that comes last. The same bits; alone, on two streams beside one
+    another, and call after call on one workspace."""
+    cfg = workloads.PrefillConfig("left", torch.bfloat16, 4, H, Hkv, D, 16, *new, *history, seed=D, value_size=512 if D == 576 else D)
+    inp = workloads.make_prefill_inputs(cfg)
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", parts)
+    want = run_paged_attention_prefill(gpu_handle, *dev, inp.scale).cpu()
+    monkeypatch.setenv("INFINIOP_AMD_PREFILL_MERGE_POLLS", polls)
+    assert torch.equal(run_paged_attention_prefill(gpu_handle, *dev, inp.scale).cpu(), want)
+
+    from infinicore_amd import ops
+    ops.clear_plan_cache()  # the knob is read when a plan is made
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = []
+    torch.cuda.synchronize()
+    for _ in range(8):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append(ops.paged_attention_prefill(*dev, None, inp.scale))
+    torch.cuda.synchronize()
+    ops.clear_plan_cache()
+    for out in outs:
+        assert torch.equal(out.cpu(), want)
 
 
 @pytest.mark.parametrize("value_size", [512, 576])
