@@ -82,14 +82,16 @@ constexpr long long kSplitTableTokens = 128; // a part per that many tokens at m
 // the kernel leaves short blocks whole and cuts middling ones into fewer parts (splitSteps).
 // Measured, us (bf16; 32 / 8 heads of 128 unless said otherwise), never split / on a table as wide as the sequence / on one
 // of 32 768 tokens; in brackets the latter two with a merge kernel of its own, which was launched wherever the table was wide:
-//   * one sequence, 3 tokens over 2 000: 33.4 / 10.2 / 9.9 (12.0, 11.8); 100 over 2 000: 36.7 / 18.0 / 17.9 (20.0, 17.8),
-//     over 500: 14.8 / 14.9 / 13.9 (14.7, 14.5); four of 64 over 5 000: 82 / 44 / 42 (42, 41); 16 of 5 over 2 000: 35.4 /
-//     29.2 / 29.5 (28.5, 28.1)
-//   * 16 heads of 64, four of 64 over 2 000: 31.5 / 18.0 / 18.0 (19.6, 18.5); 28 / 4 heads of 256, one of 100 over 2 000:
-//     50.0 / 28.0 / 27.3 (28.6, 25.0); 16 latent heads, one of 3 over 2 000: 91 / 20.4 / 20.1 (20.1, 20.1), 16 of 5: 96 / 31.1 / 30.9
-//   * without history, where nothing is split and the table alone says that it might be: one of 3 tokens 5.7 / 5.8 / 6.8
-//     (6.2, 9.7), one of 100 7.0 / 7.0 / 8.3 (7.5, 10.9), four of 64 6.6 / 6.6 / 7.5 (6.8, 12.9), 16 of 5 6.6 / 6.4 / 7.4 (6.5, 11.5)
-// What such a call still pays, about 1 us, is workgroups that look the batch up and leave.
+//   * one sequence, 3 tokens over 2 000: 33.5 / 10.0 / 9.9 (12.0, 11.8); 100 over 2 000: 37.1 / 18.4 / 18.2 (20.0, 17.8); four
+//     of 64 over 5 000: 83 / 42 / 42 (42, 41); 16 of 5 over 2 000: 34.9 / 29.7 / 29.5 (28.5, 28.1)
+//   * 16 heads of 64, four of 64 over 2 000: 31.3 / 17.9 / 17.6 (19.6, 18.5); 28 / 4 heads of 256, one of 100 over 2 000:
+//     50.6 / 27.3 / 26.8 (28.6, 25.0); 16 latent heads, one of 3 over 2 000: 90 / 19.8 / 19.5 (20.1, 20.1), 16 of 5: 97 / 30.7 / 30.3
+//   * round the length that it pays from, one of 100 over 500: 14.8 / 14.8 / 16.2 (14.7, 14.5), over 600 15.8 / 15.8 / 14.3, over
+//     700 17.5 / 15.2 / 14.9; four of 64 over 700 17.0 / 16.9 / 18.4, over 1 000 21.7 / 21.7 / 21.7; latent, one of 20 over 100
+//     15.7 / 15.7 / 17.2, over 200 20.0 / 20.0 / 18.2, over 400 28.2 / 18.5 / 18.4
+//   * without history, where nothing is split and the table alone says that it might be: one of 3 tokens 5.9 / 6.0 / 6.5
+//     (6.2, 9.7), one of 100 7.5 / 7.4 / 8.1 (7.5, 10.9), four of 64 6.5 / 6.6 / 7.2 (6.8, 12.9), 16 of 5 6.2 / 6.4 / 7.0 (6.5, 11.5)
+// What such a call still pays, 0.6 - 1.5 us, is workgroups that look the batch up and leave.
 inline void planSplit(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq, Plan &plan) {
     const long long seqs = in.num_seqs > 0 ? static_cast<long long>(in.num_seqs) : 1;
     const long long kv_heads = static_cast<long long>(in.num_kv_heads);
