@@ -76,7 +76,7 @@ constexpr long long kSplitTableTokens = 128; // a part per that many tokens at m
 // How many workgroups may share the tokens of a row block of 64 rows, and what the kernel needs to settle how many do.
 // Unsplit, a call that leaves compute units idle takes as long as its longest block: `walk` microseconds for the tokens it
 // sees (measured with one block per KV head over 5 800 tokens). P parts take a P-th of that (1.4 times that where two of
-// them share a unit), 3.5 us to meet, and 0.3 us per MB of rows that they leave and that are read back. The host knows what
+// them share a unit), 2.9 us to meet, and 0.3 us per MB of rows that they leave and that are read back. The host knows what
 // the table can hold, not the lengths: it picks the P of the longest walk (among those the device holds beside one another)
 // if that takes a fifth off it, and hands on the tokens from which a block gains at all and what a part costs, so that
 // the kernel leaves short blocks whole and cuts middling ones into fewer parts (splitSteps).
@@ -86,8 +86,8 @@ constexpr long long kSplitTableTokens = 128; // a part per that many tokens at m
 //     of 64 over 5 000: 83 / 42 / 42 (42, 41); 16 of 5 over 2 000: 34.9 / 29.7 / 29.5 (28.5, 28.1)
 //   * 16 heads of 64, four of 64 over 2 000: 31.3 / 17.9 / 17.6 (19.6, 18.5); 28 / 4 heads of 256, one of 100 over 2 000:
 //     50.6 / 27.3 / 26.8 (28.6, 25.0); 16 latent heads, one of 3 over 2 000: 90 / 19.8 / 19.5 (20.1, 20.1), 16 of 5: 97 / 30.7 / 30.3
-//   * round the length that it pays from, one of 100 over 500: 14.8 / 14.8 / 16.2 (14.7, 14.5), over 600 15.8 / 15.8 / 14.3, over
-//     700 17.5 / 15.2 / 14.9; four of 64 over 700 17.0 / 16.9 / 18.4, over 1 000 21.7 / 21.7 / 21.7; latent, one of 20 over 100
+//   * round the length that it pays from, one of 100 over 400: 12.8 / 12.9 / 14.3, over 500 14.5 / 14.7 / 14.8 (14.7, 14.5),
+//     over 600 15.7 / 15.6 / 14.2, over 700 17.5 / 14.6 / 15.0; four of 64 over 700 17.0 / 17.0 / 18.6, over 1 000 21.8 / 21.8 / 22.6; latent, one of 20 over 100
 //     15.7 / 15.7 / 17.2, over 200 20.0 / 20.0 / 18.2, over 400 28.2 / 18.5 / 18.4
 //   * without history, where nothing is split and the table alone says that it might be: one of 3 tokens 5.9 / 6.0 / 6.5
 //     (6.2, 9.7), one of 100 7.5 / 7.4 / 8.1 (7.5, 10.9), four of 64 6.5 / 6.6 / 7.2 (6.8, 12.9), 16 of 5 6.2 / 6.4 / 7.0 (6.5, 11.5)
@@ -95,7 +95,11 @@ constexpr long long kSplitTableTokens = 128; // a part per that many tokens at m
 inline void planSplit(const PagedAttentionPrefillInfo &in, const device::amd::DeviceInfo &dev, long long rows_per_seq, Plan &plan) {
     const long long seqs = in.num_seqs > 0 ? static_cast<long long>(in.num_seqs) : 1;
     const long long kv_heads = static_cast<long long>(in.num_kv_heads);
-    const long long blocks = seqs * ((rows_per_seq + 63) / 64) * kv_heads;
+    // Row blocks: of equal sequences, or half a block more for each than its rows if that is more. (Two of 137 and 92 rows are
+    // five blocks, not twice the two of 114.5: with parts for four, some wait for a second round, 28.6 us instead of 24.9
+    // over 5 531 and 3 798 at 8 heads; 16 latent heads, 33 and 30 tokens over 6 920 and 4 337, 51.5 instead of 46.4.)
+    const long long ragged = seqs == 1 || rows_per_seq % 64 == 0 ? 0 : (rows_per_seq * seqs + 32 * seqs + 63) / 64;
+    const long long blocks = kv_heads * std::max(seqs * ((rows_per_seq + 63) / 64), ragged);
     const long long tokens = static_cast<long long>(in.max_num_blocks_per_seq) * static_cast<long long>(in.page_block_size);
     const long long slots = static_cast<long long>(dev.compute_units) * (in.head_size <= 192 ? 2 : 1);
     plan.max_parts = 1;
@@ -107,7 +111,7 @@ inline void planSplit(const PagedAttentionPrefillInfo &in, const device::amd::De
     const double us_per_token = 1e-3 * (in.head_size == 64 ? 11 : in.head_size == 128 ? 14 : in.head_size == 192 ? 22
                                       : in.head_size == 256 ? 20 : 41);
     const double row_bytes = static_cast<double>(rows_per_seq) * seqs * kv_heads * in.value_size * sizeof(float);
-    const double meet_cost = 3.5, part_cost = 0.3e-6 * row_bytes;
+    const double meet_cost = 2.9, part_cost = 0.3e-6 * row_bytes;
     // time of the best split of a walk of `t` tokens
     auto split = [&](double t, int &best) {
         double least = 1e30;
@@ -127,7 +131,7 @@ inline void planSplit(const PagedAttentionPrefillInfo &in, const device::amd::De
     plan.max_parts = best;
     long long from = kSplitTableTokens;
     while (from < tokens && split(static_cast<double>(from), any) >= us_per_token * static_cast<double>(from)) {
-        from += 64;
+        from += 32;
     }
     plan.split_from = static_cast<int>(from);
     plan.part_cost = static_cast<float>(part_cost / us_per_token);
