@@ -25,10 +25,17 @@
 //   S[token][row] = K . Q^T   16 x v_mfma_f32_16x16x32 (A = K tile from LDS, B = Q held in registers
 //                             for the whole kernel; lane holds S[16T + 4g + 0..3][row c], T = 0..3)
 //   causal mask (only in steps that touch the diagonal), online softmax in fp32 / log2 domain
-//   O[row][dim] += P . V      16 x v_mfma_f32_16x16x32 (A = P rounded to the storage dtype, straight
-//                             from the registers S came out in; B = V from LDS; lane holds
-//                             O[row 4g + 0..3][16 e + c], e = 0..7)
-//   l[row]      += P . 1       2 x v_mfma_f32_16x16x32: the denominator sums the rounded probabilities
+//   O[dim][row] += V . P      16 x v_mfma_f32_16x16x32 (A = V from LDS; B = P rounded to the storage dtype, straight
+//                             from the registers S came out in; lane holds O[16 e + 4g + 0..3][row c], e = 0..7)
+//   l[row]      += 1 . P       2 x v_mfma_f32_16x16x32: the denominator sums the rounded probabilities
+//   (Where kByRow says so the operands go the other way round, and a lane holds O[row 4g + 0..3][16 e + c].)
+// A lane that holds the accumulators of one row has that row's factors at hand, and four consecutive columns of it: a rescale
+// takes no lane permutes and the output rows pass through LDS as 8-byte pieces. With four rows of one column per lane
+// (32 two-byte stores per 16 rows and lane) it was, us, 32 / 8 heads: four prompts of 1 024 - 3 072 155.0 -> 151.0; 16 chunks of 128 -
+// 512 over 1 024 - 8 192 380.7 -> 376.9, heads of 192 450 -> 441, of 256 540 -> 532; ALiBi, four of 500 - 1 500 62.0 -> 58.3; eight of
+// 100 - 400 20.9 -> 20.0. Rows that leave as parts keep that layout: 16 lanes then write 256 contiguous bytes of a row, with
+// four lanes to a row 64 (16 latent heads, eight sequences of 5 over 2 000: 26.0 against 27.5); and so do heads of 576, whose
+// results are the bits of prefill_latent.h (in fp16 the two orders round differently, equally far from 64 bits).
 // K/V fragments read from LDS are shared by the R column groups of a wavefront. A step whose tokens
 // lie beyond everything a wavefront's rows may see is skipped by that wavefront (it still takes part
 // in the copy).
@@ -509,10 +516,11 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         }
     };
     // ---- softmax state ----
-    // o[r][e][rr] = O[row 4g+rr of group r][column 16 e + c]; ol[r][rr] = sum of that row's probabilities
-    // (computed by the matrix unit as P . 1, so it sums exactly the rounded probabilities the numerator
-    // used and already sits in the accumulators' row layout); m[r] = running maximum of row c, in units
-    // of the raw dot product when there is no ALiBi (scale > 0 keeps the order), else of the scaled score.
+    // o[r][e][rr] = O[row c of group r][column 16 e + 4g + rr]; ol[r][0 .. 3] = sum of that row's probabilities (computed
+    // by the matrix unit as 1 . P, so it sums exactly the rounded probabilities the numerator used). kByRow: O[row 4g + rr of
+    // group r][column 16 e + c], and ol[r][rr] = sum of that row. m[r] = running maximum of row c, in units of the raw dot
+    // product when there is no ALiBi (scale > 0 keeps the order), else of the scaled score.
+    constexpr bool kByRow = SPLIT || KHEAD == 576;
     f32x4 o[R][G::kColsV], ol[R];
     float m[R];
     float shift[R]; // -m[r] in log2 units (0 while m[r] = -inf): what the exponent of a probability adds to its score
@@ -637,18 +645,25 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
             if (__builtin_amdgcn_ballot_w64(mx > m[r] + lazy) != 0) { // some lane's maximum, hence some row's
                 mx = maxAcrossTokenGroups(mx);
                 const float m_new = maxOf(m[r], mx);
-                // rescale. Lane holds accumulators of rows 4g..4g+3, whose factors live in lanes 4g..4g+3.
                 const float alpha = m_new > m[r] ? fastExp2((m[r] - m_new) * unit) : 1.0f;
                 m[r] = m_new;
                 // a row that has seen nothing yet keeps m = -inf: subtract 0, p = 2^-inf = 0
                 shift[r] = m_new == -INFINITY ? 0.0f : -m_new * unit;
+                if constexpr (kByRow) { // the factors of rows 4g..4g+3 live in lanes 4g..4g+3
 #pragma unroll
-                for (int rr = 0; rr < 4; ++rr) {
-                    const float alpha_r = __shfl(alpha, 4 * g + rr, 64);
-                    ol[r][rr] *= alpha_r;
+                    for (int rr = 0; rr < 4; ++rr) {
+                        const float alpha_r = __shfl(alpha, 4 * g + rr, 64);
+                        ol[r][rr] *= alpha_r;
+#pragma unroll
+                        for (int e = 0; e < G::kColsV; ++e) {
+                            o[r][e][rr] *= alpha_r;
+                        }
+                    }
+                } else {
+                    ol[r] *= alpha;
 #pragma unroll
                     for (int e = 0; e < G::kColsV; ++e) {
-                        o[r][e][rr] *= alpha_r;
+                        o[r][e] *= alpha;
                     }
                 }
             }
@@ -697,13 +712,13 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
             if (e == 0) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
-                    ol[r] = T::mfmaK32(p_op[r][u], ones, ol[r]);
+                    ol[r] = kByRow ? T::mfmaK32(p_op[r][u], ones, ol[r]) : T::mfmaK32(ones, p_op[r][u], ol[r]);
                 }
                 __builtin_amdgcn_sched_group_barrier(0x008, R, 0);
             }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                o[r][e] = T::mfmaK32(p_op[r][u], cur, o[r][e]);
+                o[r][e] = kByRow ? T::mfmaK32(p_op[r][u], cur, o[r][e]) : T::mfmaK32(cur, p_op[r][u], o[r][e]);
             }
             __builtin_amdgcn_sched_group_barrier(0x008, R, 0);
         }
@@ -743,20 +758,31 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         }
     }
 
-    // ---- normalise and store. A lane holds single columns (16 e + c) of its rows; the wavefront's 16 R rows pass
-    // through LDS (the tile buffers: every wavefront is past the last barrier of the loop, nothing is in flight) and go
-    // out as 16-byte pieces, 64 lanes on consecutive pieces ----
+    // ---- normalise and store. A lane holds four consecutive columns (16 e + 4g ..) of row c of a group; the wavefront's
+    // 16 R rows pass through LDS (the tile buffers: every wavefront is past the last barrier of the loop, nothing is in
+    // flight; 16-byte pieces swizzled by the row, so that neither the writes of 16 rows nor the reads meet in a bank) and
+    // go out as 16-byte pieces, 64 lanes on consecutive pieces ----
     static_assert(sizeof(Tiles) >= 4 * R * 16 * VHEAD * 2, "the tile buffers hold the output rows of all four wavefronts");
-    unsigned short *stage = reinterpret_cast<unsigned short *>(&tiles) + w * (R * 16 * VHEAD);
+    constexpr int kSwizzleV = G::kChunksPerRowV % 16 == 0 ? 16 : 8;
+    auto pieceOf = [](int row, int chunk) { return row * G::kChunksPerRowV + (chunk ^ (row & (kSwizzleV - 1))); };
+    uint4 *stage = reinterpret_cast<uint4 *>(&tiles) + w * (R * 16 * G::kChunksPerRowV);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
+        if constexpr (kByRow) { // single columns (16 e + c) of rows 4g..4g+3
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const float inv_l = 1.0f / (ol[r][rr] + 1e-6f);
-            unsigned short *row = stage + (r * 16 + 4 * g + rr) * VHEAD + c;
+            for (int rr = 0; rr < 4; ++rr) {
+                const float inv_l = 1.0f / (ol[r][rr] + 1e-6f);
+#pragma unroll
+                for (int e = 0; e < G::kColsV; ++e) {
+                    reinterpret_cast<unsigned short *>(stage + pieceOf(r * 16 + 4 * g + rr, 2 * e + (c >> 3)))[c & 7] = static_cast<unsigned short>(T::pack2(o[r][e][rr] * inv_l, 0.0f));
+                }
+            }
+        } else {
+            const float inv_l = 1.0f / (ol[r][0] + 1e-6f);
 #pragma unroll
             for (int e = 0; e < G::kColsV; ++e) {
-                row[16 * e] = static_cast<unsigned short>(T::pack2(o[r][e][rr] * inv_l, 0.0f));
+                const f32x4 x = o[r][e] * inv_l;
+                reinterpret_cast<uint2 *>(stage + pieceOf(r * 16 + c, 2 * e + (g >> 1)))[g & 1] = make_uint2(T::pack2(x[0], x[1]), T::pack2(x[2], x[3]));
             }
         }
     }
@@ -777,7 +803,7 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
             continue;
         }
         const int head = kv_head * a.group + (row - token * a.group);
-        const uint4 x = *reinterpret_cast<const uint4 *>(stage + local_row * VHEAD + 8 * chunk);
+        const uint4 x = stage[pieceOf(local_row, chunk)];
         S *o_ptr = static_cast<S *>(a.out) + (span.q_start + token) * a.o_stride + head * a.o_head_stride;
         *reinterpret_cast<uint4 *>(o_ptr + 8 * chunk) = x;
     }
