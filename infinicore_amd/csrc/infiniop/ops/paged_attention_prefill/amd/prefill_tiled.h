@@ -308,41 +308,9 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         partial = split.used > 1;
     }
 
-    // ---- this lane's columns: row c of each of the wavefront's R column groups ----
-    uint4 q_reg[R][G::kLoadsK];
-    int visible[R];
-    float slope[R];
-    int wave_max_visible = 0, wave_min_visible = 0x7fffffff;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int row = block_row0 + (w * R + r) * 16 + c;
-        const bool valid = row < total_rows;
-        const int token = valid ? row / a.group : 0;
-        const int head = kv_head * a.group + (valid ? row - token * a.group : 0);
-        visible[r] = valid ? visibleTokens(span, token) : 0;
-        slope[r] = (a.alibi_slopes != nullptr && valid) ? a.alibi_slopes[head] * kLog2e : 0.0f;
-        const S *q_ptr = static_cast<const S *>(a.q) + (span.q_start + token) * a.q_stride + head * a.q_head_stride;
-#pragma unroll
-        for (int kk = 0; kk < G::kLoadsK; ++kk) {
-            q_reg[r][kk] = valid ? *reinterpret_cast<const uint4 *>(q_ptr + 32 * kk + 8 * g) : make_uint4(0, 0, 0, 0);
-        }
-        wave_max_visible = max(wave_max_visible, visible[r]);
-        wave_min_visible = min(wave_min_visible, valid ? visible[r] : 0x7fffffff);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        wave_max_visible = max(wave_max_visible, __shfl_xor(wave_max_visible, off, 64));
-        wave_min_visible = min(wave_min_visible, __shfl_xor(wave_min_visible, off, 64));
-    }
-    wave_max_visible = __builtin_amdgcn_readfirstlane(wave_max_visible);
-    wave_min_visible = __builtin_amdgcn_readfirstlane(wave_min_visible);
-
-    // ---- copy side: per step this wavefront moves one 16-token tile of K and one of V (64-token
-    // steps: tile w of both), or one tile of either (32-token steps: wavefronts 0, 1 the K tiles,
-    // wavefronts 2, 3 the V tiles) ----
-    const bool copies_k = TT == 4 || w < 2;
-    const bool copies_v = TT == 4 || w >= 2;
-    const int copy_tile = TT == 4 ? w : (w & 1);
+    // ---- page ids, asked for ahead of the query: the first tiles wait for them and for nothing else. (Behind the query, and
+    // with the visible ranges below found by permutes through the LDS unit: four prompts of 19 - 250, 32 / 8 heads of 128, 9.50 us
+    // instead of 8.97, heads of 64 7.31 / 7.08, of 192 12.1 / 11.8; eight of 100 - 400 20.0 / 19.6) ----
     const char *k_head = reinterpret_cast<const char *>(static_cast<const S *>(a.k_cache) + kv_head * a.k_head_stride);
     const char *v_head = reinterpret_cast<const char *>(static_cast<const S *>(a.v_cache) + kv_head * a.v_head_stride);
     const int64_t table_row = seq * a.block_table_batch_stride;
@@ -364,6 +332,38 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     };
     int id_batch = SPLIT ? min((first_step * BN) >> a.block_shift, last_entry) >> 6 : 0;
     int ids_cur = loadIdBatch(id_batch), ids_next = loadIdBatch(id_batch + 1);
+
+    // ---- this lane's columns: row c of each of the wavefront's R column groups ----
+    uint4 q_reg[R][G::kLoadsK];
+    int visible[R];
+    float slope[R];
+    int wave_max_visible = 0, wave_min_visible = 0x7fffffff;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = block_row0 + (w * R + r) * 16 + c;
+        const bool valid = row < total_rows;
+        const int token = valid ? row / a.group : 0;
+        const int head = kv_head * a.group + (valid ? row - token * a.group : 0);
+        visible[r] = valid ? visibleTokens(span, token) : 0;
+        slope[r] = (a.alibi_slopes != nullptr && valid) ? a.alibi_slopes[head] * kLog2e : 0.0f;
+        const S *q_ptr = static_cast<const S *>(a.q) + (span.q_start + token) * a.q_stride + head * a.q_head_stride;
+#pragma unroll
+        for (int kk = 0; kk < G::kLoadsK; ++kk) {
+            q_reg[r][kk] = valid ? *reinterpret_cast<const uint4 *>(q_ptr + 32 * kk + 8 * g) : make_uint4(0, 0, 0, 0);
+        }
+        wave_max_visible = max(wave_max_visible, visible[r]);
+        wave_min_visible = min(wave_min_visible, valid ? visible[r] : 0x7fffffff);
+    }
+    // (data-parallel moves: twelve dependent permutes through the LDS unit are as long as a memory round trip)
+    wave_max_visible = __builtin_amdgcn_readfirstlane(waveMaxInt(wave_max_visible));
+    wave_min_visible = __builtin_amdgcn_readfirstlane(-waveMaxInt(-wave_min_visible));
+
+    // ---- copy side: per step this wavefront moves one 16-token tile of K and one of V (64-token
+    // steps: tile w of both), or one tile of either (32-token steps: wavefronts 0, 1 the K tiles,
+    // wavefronts 2, 3 the V tiles) ----
+    const bool copies_k = TT == 4 || w < 2;
+    const bool copies_v = TT == 4 || w >= 2;
+    const int copy_tile = TT == 4 ? w : (w & 1);
     auto pageOfEntry = [&](int entry) {
         const int e = min(entry, last_entry);
         const int raw = (e >> 6) == id_batch ? __builtin_amdgcn_readlane(ids_cur, e & 63)
