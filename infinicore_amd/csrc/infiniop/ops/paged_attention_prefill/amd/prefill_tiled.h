@@ -310,7 +310,8 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
 
     // ---- page ids, asked for ahead of the query: the first tiles wait for them and for nothing else. (Behind the query, and
     // with the visible ranges below found by permutes through the LDS unit: four prompts of 19 - 250, 32 / 8 heads of 128, 9.50 us
-    // instead of 8.97, heads of 64 7.31 / 7.08, of 192 12.1 / 11.8; eight of 100 - 400 20.0 / 19.6) ----
+    // instead of 8.97, heads of 64 7.31 / 7.08, of 192 12.1 / 11.8; eight of 100 - 400 20.0 / 19.6. Behind it with heads of 576, 18 loads per lane:
+    // 16 latent heads, eight of 5 over 2 000, split, 26.2, ahead of it 26.5.) ----
     const char *k_head = reinterpret_cast<const char *>(static_cast<const S *>(a.k_cache) + kv_head * a.k_head_stride);
     const char *v_head = reinterpret_cast<const char *>(static_cast<const S *>(a.v_cache) + kv_head * a.v_head_stride);
     const int64_t table_row = seq * a.block_table_batch_stride;
@@ -331,7 +332,10 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
         return id;
     };
     int id_batch = SPLIT ? min((first_step * BN) >> a.block_shift, last_entry) >> 6 : 0;
-    int ids_cur = loadIdBatch(id_batch), ids_next = loadIdBatch(id_batch + 1);
+    int ids_cur = 0, ids_next = 0;
+    if constexpr (KHEAD != 576) {
+        ids_cur = loadIdBatch(id_batch), ids_next = loadIdBatch(id_batch + 1);
+    }
 
     // ---- this lane's columns: row c of each of the wavefront's R column groups ----
     uint4 q_reg[R][G::kLoadsK];
@@ -357,6 +361,9 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     // (data-parallel moves: twelve dependent permutes through the LDS unit are as long as a memory round trip)
     wave_max_visible = __builtin_amdgcn_readfirstlane(waveMaxInt(wave_max_visible));
     wave_min_visible = __builtin_amdgcn_readfirstlane(-waveMaxInt(-wave_min_visible));
+    if constexpr (KHEAD == 576) {
+        ids_cur = loadIdBatch(id_batch), ids_next = loadIdBatch(id_batch + 1);
+    }
 
     // ---- copy side: per step this wavefront moves one 16-token tile of K and one of V (64-token
     // steps: tile w of both), or one tile of either (32-token steps: wavefronts 0, 1 the K tiles,
@@ -763,7 +770,7 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     // flight; 16-byte pieces swizzled by the row, so that neither the writes of 16 rows nor the reads meet in a bank) and
     // go out as 16-byte pieces, 64 lanes on consecutive pieces ----
     static_assert(sizeof(Tiles) >= 4 * R * 16 * VHEAD * 2, "the tile buffers hold the output rows of all four wavefronts");
-    constexpr int kSwizzleV = G::kChunksPerRowV % 16 == 0 ? 16 : 8;
+    constexpr int kSwizzleV = kByRow ? 1 : (G::kChunksPerRowV % 16 == 0 ? 16 : 8); // (none for single columns: offsets are immediates)
     auto pieceOf = [](int row, int chunk) { return row * G::kChunksPerRowV + (chunk ^ (row & (kSwizzleV - 1))); };
     uint4 *stage = reinterpret_cast<uint4 *>(&tiles) + w * (R * 16 * G::kChunksPerRowV);
 #pragma unroll
