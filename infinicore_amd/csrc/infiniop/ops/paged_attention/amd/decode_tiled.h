@@ -56,6 +56,8 @@ struct TileBF16 : BFloat16 {
         f32x2 v = {lo, hi};
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
     }
+    // the products with `factor`, in fp32 and then to storage
+    static __device__ __forceinline__ uint32_t packProducts(float lo, float hi, float factor) { return pack2(lo * factor, hi * factor); }
     static __device__ __forceinline__ float unpackLo(uint32_t w) { return __uint_as_float(w << 16); }
     static __device__ __forceinline__ float unpackHi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 };
@@ -71,6 +73,15 @@ struct TileF16 : Half {
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
         f32x2 v = {lo, hi};
         return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+    }
+    // The products with `factor`, each rounded once: v_fma_mixlo_f16 and v_fma_mixhi_f16 round the exact product to fp16.
+    // Left to the compiler a pair is multiplied in fp32 and then converted, which rounds twice, a single value is not, and
+    // kernels that hold the same rows in other layouts would differ; so the empty asm hides one half from the other.
+    static __device__ __forceinline__ uint32_t packProducts(float lo, float hi, float factor) {
+        _Float16 first = static_cast<_Float16>(lo * factor);
+        asm("" : "+v"(first));
+        const f16x2 v = {first, static_cast<_Float16>(hi * factor)};
+        return __builtin_bit_cast(uint32_t, v);
     }
     static __device__ __forceinline__ float unpackLo(uint32_t w) {
         return static_cast<float>(__builtin_bit_cast(f16x2, w)[0]);

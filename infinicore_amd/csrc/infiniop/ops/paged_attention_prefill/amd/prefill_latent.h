@@ -425,7 +425,7 @@ __global__ void __launch_bounds__(kLatentThreads, 2) prefillLatentKernel(Prefill
             unsigned short *row = stage + (64 * half + 16 * i + 4 * g + rr) * VHEAD + 16 * kCols * quarter + c;
 #pragma unroll
             for (int e = 0; e < kCols; ++e) {
-                row[16 * e] = static_cast<unsigned short>(T::pack2(o[i][e][rr] * inv_l[rr], 0.0f));
+                row[16 * e] = static_cast<unsigned short>(T::packProducts(o[i][e][rr], 0.0f, inv_l[rr]));
             }
         }
     }

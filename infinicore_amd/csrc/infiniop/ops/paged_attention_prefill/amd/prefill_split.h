@@ -275,10 +275,10 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
                 const int q = chunk + 64 * k; // columns 64 (q / 16) + q % 16, + 16, + 32, + 48
                 if (side == 0 && q < kChunks) {
                     unsigned short *o = o_ptr + 64 * (q >> 4) + (q & 15);
-                    o[0] = static_cast<unsigned short>(T::pack2(sum[n][k].x * inv_l, 0.0f));
-                    o[16] = static_cast<unsigned short>(T::pack2(sum[n][k].y * inv_l, 0.0f));
-                    o[32] = static_cast<unsigned short>(T::pack2(sum[n][k].z * inv_l, 0.0f));
-                    o[48] = static_cast<unsigned short>(T::pack2(sum[n][k].w * inv_l, 0.0f));
+                    o[0] = static_cast<unsigned short>(T::packProducts(sum[n][k].x, 0.0f, inv_l));
+                    o[16] = static_cast<unsigned short>(T::packProducts(sum[n][k].y, 0.0f, inv_l));
+                    o[32] = static_cast<unsigned short>(T::packProducts(sum[n][k].z, 0.0f, inv_l));
+                    o[48] = static_cast<unsigned short>(T::packProducts(sum[n][k].w, 0.0f, inv_l));
                 }
             }
             if (lane < split.used) { // consumed: a replay of this call (same token) starts clean

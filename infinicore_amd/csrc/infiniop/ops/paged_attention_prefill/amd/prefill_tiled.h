@@ -33,9 +33,10 @@
 // takes no lane permutes and the output rows pass through LDS as 8-byte pieces. With four rows of one column per lane
 // (32 two-byte stores per 16 rows and lane) it was, us, 32 / 8 heads: four prompts of 1 024 - 3 072 155.0 -> 151.0; 16 chunks of 128 -
 // 512 over 1 024 - 8 192 380.7 -> 376.9, heads of 192 450 -> 441, of 256 540 -> 532; ALiBi, four of 500 - 1 500 62.0 -> 58.3; eight of
-// 100 - 400 20.9 -> 20.0. Rows that leave as parts keep that layout: 16 lanes then write 256 contiguous bytes of a row, with
-// four lanes to a row 64 (16 latent heads, eight sequences of 5 over 2 000: 26.0 against 27.5); and so do heads of 576, whose
-// results are the bits of prefill_latent.h (in fp16 the two orders round differently, equally far from 64 bits).
+// 100 - 400 20.9 -> 20.0. Kernels that may split (SPLIT) keep that layout, also for blocks that stay whole: of a part, 16 lanes then write 256
+// contiguous bytes of a row, with four lanes to a row 64 (16 latent heads, eight sequences of 5 over 2 000: 26.0 against 27.5);
+// and so do heads of 576, as prefill_latent.h does. The two layouts give the same bits: the same products are added in the same
+// order and every output is rounded once (packProducts), so that a call's table width and workspace decide about time alone.
 // K/V fragments read from LDS are shared by the R column groups of a wavefront. A step whose tokens
 // lie beyond everything a wavefront's rows may see is skipped by that wavefront (it still takes part
 // in the copy).
@@ -781,15 +782,16 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
                 const float inv_l = 1.0f / (ol[r][rr] + 1e-6f);
 #pragma unroll
                 for (int e = 0; e < G::kColsV; ++e) {
-                    reinterpret_cast<unsigned short *>(stage + pieceOf(r * 16 + 4 * g + rr, 2 * e + (c >> 3)))[c & 7] = static_cast<unsigned short>(T::pack2(o[r][e][rr] * inv_l, 0.0f));
+                    reinterpret_cast<unsigned short *>(stage + pieceOf(r * 16 + 4 * g + rr, 2 * e + (c >> 3)))[c & 7] = static_cast<unsigned short>(T::packProducts(o[r][e][rr], 0.0f, inv_l));
                 }
             }
         } else {
             const float inv_l = 1.0f / (ol[r][0] + 1e-6f);
 #pragma unroll
             for (int e = 0; e < G::kColsV; ++e) {
-                const f32x4 x = o[r][e] * inv_l;
-                reinterpret_cast<uint2 *>(stage + pieceOf(r * 16 + c, 2 * e + (g >> 1)))[g & 1] = make_uint2(T::pack2(x[0], x[1]), T::pack2(x[2], x[3]));
+                const f32x4 x = o[r][e];
+                reinterpret_cast<uint2 *>(stage + pieceOf(r * 16 + c, 2 * e + (g >> 1)))[g & 1] =
+                    make_uint2(T::packProducts(x[0], x[1], inv_l), T::packProducts(x[2], x[3], inv_l));
             }
         }
     }

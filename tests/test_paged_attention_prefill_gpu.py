@@ -363,6 +363,23 @@ def test_split_row_blocks(gpu_handle, oracle, monkeypatch, D, H, Hkv, bs, dtype,
     run_case(gpu_handle, oracle, inp, alibi=torch.tensor([2.0 ** -(i % 5 + 1) for i in range(H)]), index_dtype=idx)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,H,Hkv", [(64, 16, 4), (128, 8, 2), (192, 6, 6), (256, 14, 2), (576, 16, 1)])
+def test_whole_blocks_are_the_same_bits_in_a_kernel_that_may_split(gpu_handle, monkeypatch, D, H, Hkv, dtype):
+    """Whether a call may split depends on the width of its block table and on its workspace. Blocks of up to 100 tokens stay
+    whole (a part has 128), and the two kernels hold their accumulators in different layouts: every value is rounded once in
+    either, slopes or none."""
+    cfg = workloads.PrefillConfig(f"whole{D}", dtype, 6, H, Hkv, D, 16, 1, 100, 0, 0, seed=D, value_size=512 if D == 576 else D)
+    inp = workloads.make_prefill_inputs(cfg)
+    dev = [t.to(DEV) for t in (inp.q, inp.k_cache, inp.v_cache, inp.block_tables, inp.seq_lens, inp.cum_seq_lens_q)]
+    for alibi in (None, torch.tensor([2.0 ** -(i % 5 + 1) for i in range(H)], device=DEV)):
+        got = []
+        for parts in ("1", "4"):
+            monkeypatch.setenv("INFINIOP_AMD_PREFILL_PARTS", parts)
+            got.append(run_paged_attention_prefill(gpu_handle, *dev, inp.scale, alibi=alibi).cpu())
+        assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("polls", ["0", "3"])
 @pytest.mark.parametrize("D,H,Hkv,new,history,parts", [
     (64, 10, 2, (1, 40), (300, 1300), "5"), (128, 32, 8, (60, 70), (2000, 2100), "4"), (192, 6, 6, (1, 150), (100, 900), "7"),
