@@ -38,6 +38,8 @@
 #ifndef INFINICORE_AMD_PA_DECODE_MLA_H
 #define INFINICORE_AMD_PA_DECODE_MLA_H
 
+#include <utility>
+
 #include "decode_tiled.h"
 
 namespace op::paged_attention::amd {
@@ -395,9 +397,11 @@ __device__ __forceinline__ void softmaxStepPair(f32x4 (&o)[COLS], float &m, floa
 //   * partition size of the call: among the planned size and larger ones, in steps of 64 tokens up to what
 //     one page-id load covers (64 pages) or 1024 tokens, the one that needs the fewest tiles in a row,
 //     i.e. (rounds of workgroups) x (tiles per partition); ties go to the larger size (fewer partial
-//     results). A lane per size: one size after the other, each with a sum over the lanes, held up every workgroup
-//     of a call on new lengths by up to 3.4 us (32 sequences of 512 - 4 096, other lengths in every call: 16 heads
-//     44.2 us instead of 40.9, 128 heads 66.3 / 64.4);
+//     results). All sizes at once, a lane per size in each row of 16 lanes, every row over its own sixteen lengths: the
+//     search holds up every workgroup of a call on new lengths. us with other lengths in every call, sizes one after the
+//     other / a lane per size over all lengths of the batch / as here: 32 sequences of 512 - 4 096 with 16 heads 42.7 /
+//     38.9 / 37.6, with 128 heads 55.4 / 53.0 / 51.4; 128 of 200 - 2 000 with 128 heads 103.8 / 103.3 / 100.1; 256 of 100 -
+//     1 000 with 128 heads 105.4 / 107.0 / 102.9; 256 of 500 - 1 500 with 32 heads 145.3 / 147.9 / 141.3;
 //   * the (sequence, partition) units are numbered densely; linear workgroup id = 8 streams (u / 8) +
 //     8 stream + u % 8, so the units that exist come first, the dies get equal shares, and the workgroups
 //     of one unit (one per group of head chunks) sit on the same die and meet in its L2.
@@ -406,6 +410,18 @@ struct WidePlan {
     int seq, part, stream; // this workgroup's unit; seq < 0: none
     int len;               // length of that sequence, clamped to [0, what its block-table row can hold]
 };
+
+// Partitions of `size` tokens of a sequence: ceil(len / size) as floor((len + size - 1/2) / size), which is at least 1 / (2 size)
+// from a whole number, further than the reciprocal and the product are off (lengths above 2^21 only blunt the estimate); none of
+// length 0.
+__device__ __forceinline__ float partitionsOf(float len, float size, float inv) { return floorf((len + (size - 0.5f)) * inv); }
+// ... of the sixteen sequences whose lengths this lane's row of 16 lanes holds: they come by as rotations of the row
+template <int... J>
+__device__ __forceinline__ float partitionsOfRow(float len, float size, float inv, std::integer_sequence<int, J...>) {
+    const int x = static_cast<int>(__float_as_uint(len));
+    return partitionsOf(len, size, inv)
+         + (partitionsOf(__uint_as_float(__builtin_amdgcn_update_dpp(x, x, 0x121 + J, 0xf, 0xf, false)), size, inv) + ...); // row_ror:J + 1
+}
 
 template <typename Tindex>
 __device__ __forceinline__ WidePlan planWide(const DecodeArgs &a, int lane, int streams, int linear_id) {
@@ -429,28 +445,20 @@ __device__ __forceinline__ WidePlan planWide(const DecodeArgs &a, int lane, int 
     }
     // The search: cost(p) = (rounds of workgroups) x (tiles per partition).
     const int cap = min(64 << a.block_shift, 1024);
-    auto roundsAt = [&](int p) {
-        // partitions of this lane's sequences: ceil(len / p) through the reciprocal, corrected to be exact
-        // (lengths above 2^24 are rounded, which only blunts the estimate)
-        const float pf = static_cast<float>(p), inv = 1.0f / pf;
-        int x = 0;
+    const float compute_units = static_cast<float>(a.compute_units), compute_units_inv = __builtin_amdgcn_rcpf(compute_units);
+    auto roundsOf = [&](float units) { return partitionsOf(units * static_cast<float>(streams), compute_units, compute_units_inv); };
+    const float planned = static_cast<float>(a.partition_tokens), planned_inv = __builtin_amdgcn_rcpf(planned);
+    float planned_units = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (i >= slots) {
-                break;
-            }
-            const float lf = static_cast<float>(lens[i]);
-            float q = floorf(lf * inv);
-            q = q * pf > lf ? q - 1.0f : q;          // one too many
-            q = (q + 1.0f) * pf <= lf ? q + 1.0f : q; // one too few
-            x += static_cast<int>(q) + (q * pf < lf ? 1 : 0);
+    for (int i = 0; i < 4; ++i) {
+        if (i >= slots) {
+            break;
         }
-        const int workgroups = __builtin_amdgcn_readlane(waveInclusiveSum(x), 63) * streams;
-        return (workgroups + a.compute_units - 1) / a.compute_units;
-    };
-    const int first_rounds = roundsAt(a.partition_tokens);
+        planned_units += partitionsOf(static_cast<float>(lens[i]), planned, planned_inv);
+    }
+    const float first_rounds = roundsOf(static_cast<float>(__builtin_amdgcn_readlane(waveInclusiveSum(static_cast<int>(planned_units)), 63)));
     // (one round at the planned size: everything runs at once, larger partitions only take longer)
-    if (first_rounds > 1 && a.partition_tokens + 64 <= cap) {
+    if (first_rounds > 1.0f && a.partition_tokens + 64 <= cap) {
         // The rest of the search is the same for every call on the same lengths - the layers of a model's decode
         // step, one after the other - so its result is remembered beside the partition size left for the merge
         // kernel: one 64-bit word, a 56-bit hash of everything the search looks at above the size in units of 64
@@ -478,30 +486,19 @@ __device__ __forceinline__ WidePlan planWide(const DecodeArgs &a, int lane, int 
         if ((seen & ~0xffull) == key && a.partition_tokens + 64 * seen_steps <= cap) {
             plan.partition_tokens = a.partition_tokens + 64 * seen_steps;
         } else {
-            // a lane per size, all at once
-            const int size = a.partition_tokens + 64 * lane;
-            // ceil(len / size) as floor((len + size - 1/2) / size): at least 1 / (2 size) from a whole number, further than
-            // the reciprocal and the product are off (lengths above 2^21 only blunt the estimate)
-            const float inv = 1.0f / static_cast<float>(size), up = static_cast<float>(size) - 0.5f;
+            // Lane 16 r + i prices size i (at most sixteen: from 64 tokens to 1024) over the lengths that row r of the lanes
+            // holds, which come by as rotations of the row; then a sum across the rows.
+            const int size = a.partition_tokens + 64 * (lane & 15);
+            const float inv = __builtin_amdgcn_rcpf(static_cast<float>(size));
             float units = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (i >= slots) {
-                    break;
-                }
-                const uint32_t len = __float_as_uint(static_cast<float>(lens[i])); // 0 beyond the last sequence: no unit
-                const int count = min(a.num_seqs - 64 * i, 64);
-                for (int j = 0; j < count; j += 8) {
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        units += floorf((__uint_as_float(__builtin_amdgcn_readlane(len, (j + k) & 63)) + up) * inv);
-                    }
-                }
+            for (int i = 0; i < slots; ++i) {
+                const float len = static_cast<float>(i == 0 ? lens[0] : i == 1 ? lens[1] : i == 2 ? lens[2] : lens[3]);
+                units += partitionsOfRow(len, static_cast<float>(size), inv, std::make_integer_sequence<int, 15>{});
             }
-            const int rounds = static_cast<int>((static_cast<int64_t>(units) * streams + a.compute_units - 1) / a.compute_units);
+            const int rounds = static_cast<int>(fminf(roundsOf(sumAcrossTokenGroups(units)), 0xfffff));
             // the least cost; ties go to the larger size (fewer partial results)
-            const int cost = size <= cap ? min(rounds, 0xfffff) * ((size + kMlaWideTileTokens - 1) / kMlaWideTileTokens) : 0x1ffffff;
-            plan.partition_tokens = a.partition_tokens + 64 * (waveMaxInt(lane - 64 * cost) & 63);
+            const int cost = size <= cap ? rounds * ((size + kMlaWideTileTokens - 1) / kMlaWideTileTokens) : 0x1ffffff;
+            plan.partition_tokens = a.partition_tokens + 64 * (waveMaxInt((lane & 15) - 64 * cost) & 15);
             if (linear_id == 0 && lane == 0) {
                 *remembered = key | static_cast<unsigned long long>((plan.partition_tokens - a.partition_tokens) / 64);
             }
@@ -539,31 +536,33 @@ __device__ __forceinline__ WidePlan planWide(const DecodeArgs &a, int lane, int 
 template <typename Tindex>
 __device__ __forceinline__ bool locateWideUnit(const DecodeArgs &a, int lane, int groups_of_chunks, int &seq, int &part,
                                                int &stream, int &partition_tokens, int &len) {
-    if (a.chosen_partition != nullptr) {
-        // planned per call (see planWide): one-dimensional grid
-        const WidePlan plan = planWide<Tindex>(a, lane, a.num_kv_heads * groups_of_chunks, static_cast<int>(blockIdx.x));
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            a.chosen_partition[0] = plan.partition_tokens; // for the merge kernel
-        }
-        if (plan.seq < 0) {
-            return false;
-        }
-        // wave-uniform by construction; saying so keeps the address arithmetic in scalar registers
-        seq = __builtin_amdgcn_readfirstlane(plan.seq);
-        part = __builtin_amdgcn_readfirstlane(plan.part);
-        stream = __builtin_amdgcn_readfirstlane(plan.stream);
-        partition_tokens = __builtin_amdgcn_readfirstlane(plan.partition_tokens);
-        len = __builtin_amdgcn_readfirstlane(plan.len); // the plan has read it already: no second round trip
+    if (__builtin_expect(a.chosen_partition == nullptr, 1)) {
+        // fixed partitions on a three-dimensional grid, rotated as in decodeMlaKernel. (First, ahead of the planning code:
+        // these calls are short, and their instructions come out of a cold cache. Seven sequences of 20 tokens, 64 heads,
+        // 13.2 us behind it, 13.05 here; planned calls are no slower.)
+        seq = blockIdx.z;
+        part = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
+        stream = blockIdx.y;
+        partition_tokens = a.partition_tokens;
+        const int64_t len64 = loadIndex<Tindex>(a.seq_lens, seq);
+        const int64_t max_len = static_cast<int64_t>(a.max_blocks_per_seq) << a.block_shift;
+        len = static_cast<int>(len64 < max_len ? len64 : max_len);
         return true;
     }
-    // fixed partitions on a three-dimensional grid, rotated as in decodeMlaKernel
-    seq = blockIdx.z;
-    part = static_cast<int>((blockIdx.x + blockIdx.z) % gridDim.x);
-    stream = blockIdx.y;
-    partition_tokens = a.partition_tokens;
-    const int64_t len64 = loadIndex<Tindex>(a.seq_lens, seq);
-    const int64_t max_len = static_cast<int64_t>(a.max_blocks_per_seq) << a.block_shift;
-    len = static_cast<int>(len64 < max_len ? len64 : max_len);
+    // planned per call (see planWide): one-dimensional grid
+    const WidePlan plan = planWide<Tindex>(a, lane, a.num_kv_heads * groups_of_chunks, static_cast<int>(blockIdx.x));
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        a.chosen_partition[0] = plan.partition_tokens; // for the merge kernel
+    }
+    if (plan.seq < 0) {
+        return false;
+    }
+    // wave-uniform by construction; saying so keeps the address arithmetic in scalar registers
+    seq = __builtin_amdgcn_readfirstlane(plan.seq);
+    part = __builtin_amdgcn_readfirstlane(plan.part);
+    stream = __builtin_amdgcn_readfirstlane(plan.stream);
+    partition_tokens = __builtin_amdgcn_readfirstlane(plan.partition_tokens);
+    len = __builtin_amdgcn_readfirstlane(plan.len); // the plan has read it already: no second round trip
     return true;
 }
 

@@ -1111,42 +1111,51 @@ def test_full_size_linearity_in_v(gpu_handle):
     assert torch.all((ab - (a + b)).abs() <= 2 * ATOL + RTOL * (a + b).abs())
 
 
-@pytest.mark.parametrize("seqs, heads, lengths", [
-    (24, 128, (600, 2500)),   # one slot of lengths
-    (64, 64, (300, 3000)),    # a full slot
-    (70, 128, (700, 1100)),   # two slots, the second nearly empty
-    (200, 64, (1, 900)),      # four
-    (256, 32, (1000, 1024)),  # all of them, equal in whole partitions
-    (32, 128, (512, 4096)),
+@pytest.mark.parametrize("seqs, heads, page, lengths", [
+    (24, 128, 16, (600, 2500)),   # one slot of lengths
+    (64, 64, 16, (2000, 4096)),   # a full slot
+    (64, 16, 16, (2000, 4096)),   # 16 heads: a workgroup per partition
+    (40, 128, 64, (1500, 2048)),
+    (70, 128, 16, (900, 1300)),   # two slots, the second nearly empty
+    (200, 64, 32, (1, 900)),      # four
+    (256, 32, 16, (1000, 1024)),  # all of them, equal in whole partitions
+    (32, 128, 16, (512, 4096)),
 ])
-def test_mla_partition_search_matches_one_size_after_the_other(gpu_handle, tmp_path, seqs, heads, lengths):
-    """The size that a call settles on (a lane per size) is the one that costs least when the sizes are tried in turn."""
+@pytest.mark.parametrize("dtype, idx", [(torch.bfloat16, torch.int64), (torch.float16, torch.int32)])
+def test_mla_partition_search_matches_one_size_after_the_other(gpu_handle, tmp_path, seqs, heads, page, lengths, dtype, idx):
+    """The size that a call settles on (lanes price all sizes at once) is the one that costs least when the sizes are tried in
+    turn: on a workspace that remembers nothing, on other lengths behind a remembered size, and on the first ones again."""
     from test_decode_plan import build_probe
 
-    inp = workloads.make_decode_inputs(mla("mla_search", torch.bfloat16, seqs, heads, 16, *lengths, seed=700 + seqs))
+    inp = workloads.make_decode_inputs(mla("mla_search", dtype, seqs, heads, page, *lengths, seed=700 + seqs))
     q, k, v, bt, sl = to_device(inp)
-    out = torch.zeros((seqs, heads, 512), dtype=torch.bfloat16, device=DEV)
+    bt, sl = bt.to(idx), sl.to(idx)
+    out = torch.zeros((seqs, heads, 512), dtype=dtype, device=DEV)
     status, op = create_paged_attention(gpu_handle, out, q, k, v, bt, sl, None, inp.scale)
     assert status == 0
     size = workspace_size_attention(op)
     ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=DEV)
-    plan = build_probe(tmp_path)(seqs, heads, 1, 576, 16, bt.shape[1], value_size=512, num_blocks=k.shape[0])
-    L.check_error(L.LIBINFINIOP.infiniopPagedAttention(op, ptr(ws), size, ptr(out), ptr(q), ptr(k), ptr(v), ptr(bt), ptr(sl), None, None))
-    torch.cuda.synchronize()
+    plan = build_probe(tmp_path)(seqs, heads, 1, 576, page, bt.shape[1], value_size=512, num_blocks=k.shape[0])
     offset = plan["acc_bytes"] + 2 * plan["ml_bytes"]
-    chosen = int(ws[offset:offset + 4].view(torch.int32).item())
-    L.check_error(L.LIBINFINIOP.infiniopDestroyPagedAttentionDescriptor(op))
     chunks = -(-heads // 16)
     per_workgroup = 1 if chunks == 1 else (8 if chunks > 4 and seqs >= 48 else 4)
     streams = -(-chunks // per_workgroup)
     units = torch.cuda.get_device_properties(0).multi_processor_count
 
-    def cost(p):
-        rounds = -(-sum(-(-n // p) for n in inp.seq_lens.tolist()) * streams // units)
-        return rounds, rounds * -(-p // 32)
+    first = inp.seq_lens.tolist()
+    other = [n - (i * 37) % (n // 4 + 1) for i, n in enumerate(first)]
+    for lens in (first, other, first):
+        def cost(p):
+            rounds = -(-sum(-(-n // p) for n in lens) * streams // units)
+            return rounds, rounds * -(-p // 32)
 
-    want = plan["partition_tokens"]
-    if cost(want)[0] > 1:
-        for p in range(want + 64, 1025, 64):
+        sl.copy_(torch.tensor(lens))
+        L.check_error(L.LIBINFINIOP.infiniopPagedAttention(op, ptr(ws), size, ptr(out), ptr(q), ptr(k), ptr(v), ptr(bt), ptr(sl), None, None))
+        torch.cuda.synchronize()
+        chosen = int(ws[offset:offset + 4].view(torch.int32).item())
+        want = plan["partition_tokens"]
+        assert cost(want)[0] > 1, "the case must make the kernel search"
+        for p in range(want + 64, 1025, 64):  # (pages have 16 tokens or more: 64 of them hold as many)
             want = p if cost(p)[1] <= cost(want)[1] else want
-    assert chosen == want
+        assert chosen == want
+    L.check_error(L.LIBINFINIOP.infiniopDestroyPagedAttentionDescriptor(op))
