@@ -155,15 +155,21 @@ __device__ __forceinline__ void compilerMemoryBarrier() { asm volatile("" ::: "m
 // Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS-unit permutes: this
 // runs at the head of every wavefront, before its first memory request can go out). Rows of 16 lanes are
 // scanned with row shifts, then lane 15 of rows 0 and 2 is added to the next row, then lane 31 to rows 2, 3.
-__device__ __forceinline__ int waveInclusiveSum(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false); // row_shr:1
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false); // row_shr:2
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false); // row_shr:4
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false); // row_shr:8
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false); // row_bcast:15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false); // row_bcast:31 into rows 2 and 3
+// (Added without a sign: hashes are summed too, whose sums wrap.)
+template <int CONTROL, int ROWS>
+__device__ __forceinline__ unsigned laneMovedBits(unsigned where_none, unsigned x) {
+    return static_cast<unsigned>(__builtin_amdgcn_update_dpp(static_cast<int>(where_none), static_cast<int>(x), CONTROL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ unsigned waveInclusiveSum(unsigned x) {
+    x += laneMovedBits<0x111, 0xf>(0, x); // row_shr:1
+    x += laneMovedBits<0x112, 0xf>(0, x); // row_shr:2
+    x += laneMovedBits<0x114, 0xf>(0, x); // row_shr:4
+    x += laneMovedBits<0x118, 0xf>(0, x); // row_shr:8
+    x += laneMovedBits<0x142, 0xa>(0, x); // row_bcast:15 into rows 1 and 3
+    x += laneMovedBits<0x143, 0xc>(0, x); // row_bcast:31 into rows 2 and 3
     return x;
 }
+__device__ __forceinline__ int waveInclusiveSum(int x) { return static_cast<int>(waveInclusiveSum(static_cast<unsigned>(x))); }
 
 // Maximum over the 64 lanes, in the same manner; every lane receives it.
 __device__ __forceinline__ int waveMaxInt(int x) {

@@ -477,8 +477,8 @@ __device__ __forceinline__ WidePlan planWide(const DecodeArgs &a, int lane, int 
             h1 += x * 0x2C1B3C6Du;
             h2 += (x ^ 0x27D4EB2Fu) * 0x165667B1u;
         }
-        h1 = static_cast<unsigned>(__builtin_amdgcn_readlane(waveInclusiveSum(static_cast<int>(h1)), 63));
-        h2 = static_cast<unsigned>(__builtin_amdgcn_readlane(waveInclusiveSum(static_cast<int>(h2)), 63));
+        h1 = __builtin_amdgcn_readlane(waveInclusiveSum(h1), 63);
+        h2 = __builtin_amdgcn_readlane(waveInclusiveSum(h2), 63);
         h1 += static_cast<unsigned>(a.partition_tokens) * 0x9E3779B1u + static_cast<unsigned>(streams) * 0x85EBCA77u;
         h2 += static_cast<unsigned>(a.num_seqs) * 0xC2B2AE3Du + static_cast<unsigned>(a.compute_units) * 0x27D4EB2Fu + static_cast<unsigned>(a.block_shift);
         const unsigned long long key = ((static_cast<unsigned long long>(h1) << 32) | h2) & ~0xffull;
