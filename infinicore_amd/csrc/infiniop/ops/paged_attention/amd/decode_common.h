@@ -182,18 +182,38 @@ __device__ __forceinline__ int waveMaxInt(int x) {
     return __builtin_amdgcn_readlane(x, 63);
 }
 
-// Sum / max over the 64 lanes of a wavefront; every lane receives the result.
+// Maximum and sum of floats, in the same manner: the merges of partial results are a few round trips long, and the six
+// dependent lane permutes of waveSum would be as long again.
+__device__ __forceinline__ float laneOf(float x, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane & 63)); }
+template <int CONTROL, int ROWS>
+__device__ __forceinline__ float laneMoved(float x, float where_none) {
+    return __uint_as_float(laneMovedBits<CONTROL, ROWS>(__float_as_uint(where_none), __float_as_uint(x)));
+}
+__device__ __forceinline__ float laneMax(float x) {
+    x = fmaxf(x, laneMoved<0x111, 0xf>(x, x));
+    x = fmaxf(x, laneMoved<0x112, 0xf>(x, x));
+    x = fmaxf(x, laneMoved<0x114, 0xf>(x, x));
+    x = fmaxf(x, laneMoved<0x118, 0xf>(x, x));
+    x = fmaxf(x, laneMoved<0x142, 0xa>(x, x));
+    x = fmaxf(x, laneMoved<0x143, 0xc>(x, x));
+    return laneOf(x, 63);
+}
+__device__ __forceinline__ float laneSum(float x) {
+    x += laneMoved<0x111, 0xf>(x, 0.0f);
+    x += laneMoved<0x112, 0xf>(x, 0.0f);
+    x += laneMoved<0x114, 0xf>(x, 0.0f);
+    x += laneMoved<0x118, 0xf>(x, 0.0f);
+    x += laneMoved<0x142, 0xa>(x, 0.0f);
+    x += laneMoved<0x143, 0xc>(x, 0.0f);
+    return laneOf(x, 63);
+}
+
+// Sum over the 64 lanes by permutes through the LDS unit, in the order of a butterfly (the element-wise kernels' dot
+// products); every lane receives the result.
 __device__ __forceinline__ float waveSum(float x) {
 #pragma unroll
     for (int offset = 32; offset > 0; offset >>= 1) {
         x += __shfl_xor(x, offset, 64);
-    }
-    return x;
-}
-__device__ __forceinline__ float waveMax(float x) {
-#pragma unroll
-    for (int offset = 32; offset > 0; offset >>= 1) {
-        x = fmaxf(x, __shfl_xor(x, offset, 64));
     }
     return x;
 }

@@ -18,6 +18,7 @@
 namespace op::paged_attention::amd {
 
 constexpr int kReduceThreads = 256;
+constexpr int kWaveMergePartitions = 8; // up to here a wavefront merges a row (decodeReduceWaveKernel)
 constexpr int kReduceRowGroups = kReduceThreads / 16;
 
 __device__ __forceinline__ float swapMax(float x) {
@@ -142,33 +143,26 @@ __global__ void __launch_bounds__(kReduceThreads) decodeReduceKernel(DecodeArgs 
     }
 }
 
-// Maximum and sum over the 64 lanes with data-parallel moves, in the manner of waveInclusiveSum (decode_common.h). Permutes
-// through the LDS unit, six dependent ones for either, a round trip each: latent decode of 32 sequences of 512 - 4 096 with
-// them here and in the hash of planWide 128 heads 64.1 us instead of 63.3, 16 heads 41.0 / 40.5.
-template <int CONTROL, int ROWS>
-__device__ __forceinline__ float laneMoved(float x, float where_none) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(where_none), __float_as_uint(x), CONTROL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ float laneMax(float x) {
-    x = fmaxf(x, laneMoved<0x111, 0xf>(x, x)); // row_shr:1
-    x = fmaxf(x, laneMoved<0x112, 0xf>(x, x)); // row_shr:2
+// Maximum and sum over lanes 0 .. 7 with data-parallel moves (decode_common.h), for every lane. Permutes through the LDS unit,
+// six dependent ones for either, are a round trip each: latent decode of 32 sequences of 512 - 4 096 with them here and in the
+// hash of planWide 128 heads 64.1 us instead of 63.3, 16 heads 41.0 / 40.5; one sequence of 400 tokens, 32 / 8 heads of 128,
+// 9.9 / 9.8. The sum adds the lanes in the order of a butterfly: (0 + 4) + (2 + 6) and (1 + 5) + (3 + 7).
+static_assert(kWaveMergePartitions == 8, "a partition per lane");
+__device__ __forceinline__ float firstLanesMax(float x) {
     x = fmaxf(x, laneMoved<0x114, 0xf>(x, x)); // row_shr:4
-    x = fmaxf(x, laneMoved<0x118, 0xf>(x, x)); // row_shr:8
-    x = fmaxf(x, laneMoved<0x142, 0xa>(x, x)); // row_bcast:15 into rows 1 and 3
-    x = fmaxf(x, laneMoved<0x143, 0xc>(x, x)); // row_bcast:31 into rows 2 and 3
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63));
+    x = fmaxf(x, laneMoved<0x112, 0xf>(x, x)); // row_shr:2
+    x = fmaxf(x, laneMoved<0x111, 0xf>(x, x)); // row_shr:1
+    return laneOf(x, kWaveMergePartitions - 1);
 }
-__device__ __forceinline__ float laneSum(float x) {
-    x += laneMoved<0x111, 0xf>(x, 0.0f);
-    x += laneMoved<0x112, 0xf>(x, 0.0f);
+__device__ __forceinline__ float firstLanesSum(float x) {
+    asm("" : "+v"(x)); // a product as it is rounded in every lane: a fused first step would round it in lanes 0 .. 3 alone
     x += laneMoved<0x114, 0xf>(x, 0.0f);
-    x += laneMoved<0x118, 0xf>(x, 0.0f);
-    x += laneMoved<0x142, 0xa>(x, 0.0f);
-    x += laneMoved<0x143, 0xc>(x, 0.0f);
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63));
+    x += laneMoved<0x112, 0xf>(x, 0.0f);
+    x += laneMoved<0x111, 0xf>(x, 0.0f);
+    return laneOf(x, kWaveMergePartitions - 1);
 }
 
-// The same merge for calls with few partitions per sequence (the host uses it up to 8): one WAVEFRONT
+// The same merge for calls with few partitions per sequence (up to kWaveMergePartitions): one WAVEFRONT
 // per (query head, sequence), four per workgroup. Lane p fetches (m, l) of partition p; the partial rows
 // are then added one after the other with every lane on its own columns (column lane * kVec + 64 kVec j:
 // every load instruction of the wavefront reads one contiguous piece of a row), all loads independent of
@@ -195,14 +189,14 @@ __global__ void __launch_bounds__(kReduceThreads) decodeReduceWaveKernel(DecodeA
     if (len <= partition_tokens) {
         return; // empty sequence, or already finished by the decode kernel (uniform for the wavefront)
     }
-    const int parts = (len + partition_tokens - 1) / partition_tokens; // <= max_partitions <= 64
+    const int parts = (len + partition_tokens - 1) / partition_tokens; // <= max_partitions <= kWaveMergePartitions
     const int64_t slot0 = pair * a.max_partitions;
 
     const float m_p = lane < parts ? a.part_m[slot0 + lane] : -INFINITY;
     const float l_p = lane < parts ? a.part_l[slot0 + lane] : 0.0f;
-    const float m = laneMax(m_p);
+    const float m = firstLanesMax(m_p);
     const float w_p = mergeWeight(m_p, m);
-    const float l = laneSum(l_p * w_p);
+    const float l = firstLanesSum(l_p * w_p);
 
     float acc[kLoads][kVec];
 #pragma unroll
@@ -220,7 +214,7 @@ __global__ void __launch_bounds__(kReduceThreads) decodeReduceWaveKernel(DecodeA
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int p = min(p0 + u, parts - 1);
-            w[u] = p0 + u < parts ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w_p), p)) : 0.0f;
+            w[u] = p0 + u < parts ? laneOf(w_p, p) : 0.0f;
             row[u] = a.part_acc + (slot0 + p) * VALUE + lane * kVec;
         }
         float v[4][kLoads][kVec];

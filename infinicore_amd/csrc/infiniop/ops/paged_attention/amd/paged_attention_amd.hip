@@ -45,7 +45,7 @@ void launchGeneric(const DecodeArgs &a, const Plan &plan, hipStream_t stream) {
 
 template <typename T, typename Tindex>
 void launchReduce(const DecodeArgs &a, hipStream_t stream) {
-    if (a.max_partitions <= 8) {
+    if (a.max_partitions <= kWaveMergePartitions) {
         // few partitions per sequence: one wavefront per (head, sequence) (up to 8: m2 14.6 -> 8.2 us; with
         // 16, of which m1 uses up to 16, the workgroup-per-row kernel is the faster one: 4.7 vs 5.4 us)
         const long long pairs = static_cast<long long>(a.num_heads) * a.num_seqs;

@@ -98,32 +98,6 @@ __device__ __forceinline__ void publishPart(const PrefillArgs &a, int64_t row0, 
     }
 }
 
-// Maximum and sum over the 64 lanes, for every lane, in the manner of waveInclusiveSum (decode_common.h): a merge is a few
-// round trips long, and the six dependent lane permutes of waveMax or waveSum per row would be as long again.
-__device__ __forceinline__ float laneOf(float x, int lane) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane & 63)); }
-template <int CONTROL, int ROWS>
-__device__ __forceinline__ float moved(float x, float where_none) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(where_none), __float_as_uint(x), CONTROL, ROWS, 0xf, false));
-}
-__device__ __forceinline__ float mergeMax(float x) {
-    x = fmaxf(x, moved<0x111, 0xf>(x, x)); // row_shr:1
-    x = fmaxf(x, moved<0x112, 0xf>(x, x)); // row_shr:2
-    x = fmaxf(x, moved<0x114, 0xf>(x, x)); // row_shr:4
-    x = fmaxf(x, moved<0x118, 0xf>(x, x)); // row_shr:8
-    x = fmaxf(x, moved<0x142, 0xa>(x, x)); // row_bcast:15 into rows 1 and 3
-    x = fmaxf(x, moved<0x143, 0xc>(x, x)); // row_bcast:31 into rows 2 and 3
-    return laneOf(x, 63);
-}
-__device__ __forceinline__ float mergeSum(float x) {
-    x += moved<0x111, 0xf>(x, 0.0f);
-    x += moved<0x112, 0xf>(x, 0.0f);
-    x += moved<0x114, 0xf>(x, 0.0f);
-    x += moved<0x118, 0xf>(x, 0.0f);
-    x += moved<0x142, 0xa>(x, 0.0f);
-    x += moved<0x143, 0xc>(x, 0.0f);
-    return laneOf(x, 63);
-}
-
 __device__ __forceinline__ unsigned long long *leftMarks(const PrefillArgs &a, int block_index, int kv_head) {
     return a.part_left + (static_cast<int64_t>(block_index) * a.num_kv_heads + kv_head) * kMergeWavefronts;
 }
@@ -227,8 +201,8 @@ __device__ __forceinline__ void mergeParts(const PrefillArgs &a, const SeqSpan &
 #pragma unroll
                 for (int n = 0; n < N; ++n) {
                     const float m = lane < seen[n] ? ml[n].x : -INFINITY;
-                    weight[n] = mergeWeight(m, mergeMax(m));
-                    l[n] = mergeSum(lane < seen[n] ? ml[n].y * weight[n] : 0.0f);
+                    weight[n] = mergeWeight(m, laneMax(m));
+                    l[n] = laneSum(lane < seen[n] ? ml[n].y * weight[n] : 0.0f);
                 }
             }
 #pragma unroll
