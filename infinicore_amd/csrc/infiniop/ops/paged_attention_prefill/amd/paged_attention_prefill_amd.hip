@@ -46,6 +46,7 @@ void launchTiledHead(const PrefillArgs &args, const Plan &plan, hipStream_t stre
     const int resident = groups == 2 ? prefillWorkgroupsPerUnit<KHEAD, 2>() : prefillWorkgroupsPerUnit<KHEAD, 1>();
     const unsigned slots = static_cast<unsigned>(plan.compute_units * resident);
     a.longest_first = longestFirst<KHEAD>(grid.x, slots) ? 1 : 0;
+    a.slots = slots;
     if constexpr (KHEAD == VHEAD && KHEAD <= 256) {
         if (groups == 2) {
             prefillTiledKernel<T, Tindex, KHEAD, VHEAD, 2, PLAIN><<<grid, kPrefillThreads, 0, stream>>>(a);

@@ -35,6 +35,7 @@ struct PrefillArgs {
     int32_t block_shift; // log2(block_size) if a power of two, else -1
     int32_t num_blocks;  // pool size; table entries are clamped into [0, num_blocks)
     int32_t max_blocks_per_seq;
+    uint32_t slots; // workgroups that the device holds at a time
 
     // element strides
     int64_t q_stride, q_head_stride;

@@ -98,6 +98,25 @@ constexpr bool longestFirst(unsigned long long grid, unsigned long long slots) {
     return (KHEAD == 64 ? 4 * grid > 7 * slots : grid > slots) && grid <= 6 * slots;
 }
 
+// Whether one of the two workgroups of a compute unit goes ahead of the other (wavefront priorities below), heads of 128. Side
+// by side the two end together and the units take up the next ones together, which is best for whole rounds. Where the last round
+// has at most one workgroup for a unit and the blocks are of much the same length, half of a round ending early lets the next
+// begin under the other half. us, side by side / ahead: 64 / 8 heads,
+// 9 sequences of 128 over 1 886 (1.1 rounds) 105.8 / 103.0, 11 (1.4) 118.2 / 108.6, 17 (2.1) 171.7 / 167.2; 9 of 512 over 512, 32 / 8
+// heads (2.2), 82.3 / 76.7; but 13 (1.6) 126.2 / 132.6, 16 (2.0) 140.7 / 150.9, 21 (2.6) 193.4 / 210.3, 33 (4.1) 333 / 345. Unequal blocks
+// end apart by themselves, longest first, which tells in the first two rounds: 9 of 128 over 1 500 - 2 300 99.0 / 95.9, over
+// 1 000 - 3 000 86.4 / 93.2; 18 over 1 000 - 3 000 171 / 169, over 600 - 3 400 the same; three prompts of 500 - 2 500 85.6 / 87.5.
+// Heads of 64 lose in all of these (9 sequences 56.7 / 59.7), larger ones have a unit to themselves.
+struct BlockLengths {
+    int blocks;      // row blocks of the call; 0 where they are not dealt longest first, or of more than 64 sequences
+    int least, most; // what the shortest sees, and more than the longest does, in blocks of tokens
+};
+constexpr bool oneAhead(BlockLengths of, unsigned kv_heads, unsigned slots) {
+    const unsigned workgroups = of.blocks * kv_heads;
+    return (workgroups > slots && 2 * workgroups <= 3 * slots && of.least >= (of.most + 1) / 2)
+        || (workgroups > 2 * slots && 2 * workgroups < 5 * slots && of.least >= (of.most + 7) / 8);
+}
+
 // Which (sequence, row block) workgroup `x` of a KV head works on: the x-th longest block of the batch. The dispatcher
 // starts workgroups in the order of their numbers, so the long blocks of a ragged batch start first and the last round
 // is made of short ones. A block's rank goes by the tokens it sees, counted in blocks of tokens (block_rows rows are
@@ -115,7 +134,7 @@ constexpr bool longestFirst(unsigned long long grid, unsigned long long slots) {
 // enough to be split (of more than 64 sequences, only that there are too many to know); below 0 is none.
 template <typename Tindex, bool ASK = false, typename Place = int>
 __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int block_rows, int x, int &seq, int &block,
-                                             SeqSpan &span_out, Place place = {}) {
+                                             SeqSpan &span_out, BlockLengths *lengths = nullptr, Place place = {}) {
     const int block_tokens = max(block_rows / a.group, 1);
     for (int base = 0; base < a.num_seqs; base += 64) {
         const int idx = base + lane;
@@ -163,6 +182,9 @@ __device__ __forceinline__ bool findRowBlock(const PrefillArgs &a, int lane, int
         // lo ends as the largest key with more than x blocks from it on; every block has at least the first lo, none hi
         int lo = __builtin_amdgcn_readfirstlane(-waveMaxInt(nb > 0 ? nb - 1 - top : -0x40000000));
         int hi = __builtin_amdgcn_readfirstlane(waveMaxInt(nb > 0 ? top : -0x40000000)) + 1;
+        if (lengths != nullptr && a.num_seqs <= 64) {
+            *lengths = {blocks, lo, hi};
+        }
         while (hi - lo > 1) { // blocksFrom(lo) > x >= blocksFrom(hi)
             const int mid = lo + (hi - lo) / 2;
             if (blocksFrom(mid) > x) {
@@ -269,13 +291,14 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     };
 
     int seq = 0, block = 0;
+    BlockLengths lengths{0, 0, 0};
     SeqSpan span;
     if constexpr (SPLIT) {
-        if (!findRowBlock<Tindex, true>(a, lane, BM, 0, seq, block, span, place)) {
+        if (!findRowBlock<Tindex, true>(a, lane, BM, 0, seq, block, span, nullptr, place)) {
             return;
         }
     } else {
-        if (!findRowBlock<Tindex>(a, lane, BM, block_index, seq, block, span)) {
+        if (!findRowBlock<Tindex>(a, lane, BM, block_index, seq, block, span, KHEAD == 128 && R == 2 ? &lengths : nullptr)) {
             return;
         }
     }
@@ -507,7 +530,8 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
     // for as long as it has vector instructions ready. The two blocks of matrix instructions of a step therefore run at
     // a higher priority than the softmax between them (a softmax then fills the issue slots that the other wavefront's
     // matrix instructions leave free), and of two wavefronts in the same kind of phase the one in the odd hardware
-    // slot goes first, which pushes the pair apart. Bit 0 of the wavefront's slot number: HW_ID bits [3:0].
+    // slot goes first, which pushes the pair apart; where oneAhead says so it goes first in its softmax as well. Bit 0 of the
+    // wavefront's slot number: HW_ID bits [3:0].
     const bool odd_slot = (__builtin_amdgcn_s_getreg((3 << 11) | 4) & 1) != 0;
     auto matrixPhase = [&]() {
         if (odd_slot) {
@@ -516,9 +540,12 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
             __builtin_amdgcn_s_setprio(2);
         }
     };
+    const bool ahead = oneAhead(lengths, a.num_kv_heads, a.slots);
     auto vectorPhase = [&]() {
         if (odd_slot) {
-            __builtin_amdgcn_s_setprio(1);
+            if (!ahead) {
+                __builtin_amdgcn_s_setprio(1);
+            }
         } else {
             __builtin_amdgcn_s_setprio(0);
         }

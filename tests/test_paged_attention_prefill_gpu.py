@@ -599,6 +599,17 @@ def test_scores_that_climb_along_the_sequence(gpu_handle, oracle, monkeypatch, g
     run_case(gpu_handle, oracle, inp)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("seqs, history", [(9, 700), (12, 700), (13, 700), (17, 130), (20, 130)])
+def test_rounds_with_one_workgroup_of_a_unit_ahead(gpu_handle, oracle, seqs, history, dtype):
+    """64 row blocks of 128 rows per sequence on 512 places: just above one and two rounds, up to half a round more, and beyond
+    it; rows of every block."""
+    inp = workloads.make_prefill_inputs(prefill_config("ahead", dtype, seqs, 64, 8, 128, 16, (128, 128), (history, history), seed=seqs))
+    grid, slots = row_block_grid(inp, 128)
+    assert grid > slots and seqs * 64 < 3 * slots
+    run_case(gpu_handle, oracle, inp, rows=[128 * s + t for s in range(seqs) for t in (0, 15, 16, 77, 127)])
+
+
 def row_block_grid(inp, rows):
     """Workgroups of a launch with `rows` rows per workgroup, and how many the device holds at a time."""
     cfg = inp.config
