@@ -795,10 +795,13 @@ __global__ void __launch_bounds__(kPrefillThreads, (prefillWorkgroupsPerUnit<KHE
 
     // ---- normalise and store. A lane holds four consecutive columns (16 e + 4g ..) of row c of a group; the wavefront's
     // 16 R rows pass through LDS (the tile buffers: every wavefront is past the last barrier of the loop, nothing is in
-    // flight; 16-byte pieces swizzled by the row, so that neither the writes of 16 rows nor the reads meet in a bank) and
-    // go out as 16-byte pieces, 64 lanes on consecutive pieces ----
+    // flight) and go out as 16-byte pieces, 64 lanes on consecutive pieces. Pieces are swizzled by the row: of values of 128 and
+    // 256 neither the writes of 16 rows nor the reads meet in a bank; of 64 and 192, where two rows share the 64 banks, the writes
+    // of rows c and c + 8 do. (Swizzled by every second row they meet nowhere: eight of 100 - 400 over up to 2 000, heads
+    // of 192, 90.5 -> 89.8 us, but four prompts of 20 - 250 11.85 -> 12.02 and five of 30 - 120 8.98 -> 9.14, where the addresses cost
+    // more; heads of 64 the same.) kByRow: single columns of four rows, not swizzled, so that offsets are immediates ----
     static_assert(sizeof(Tiles) >= 4 * R * 16 * VHEAD * 2, "the tile buffers hold the output rows of all four wavefronts");
-    constexpr int kSwizzleV = kByRow ? 1 : (G::kChunksPerRowV % 16 == 0 ? 16 : 8); // (none for single columns: offsets are immediates)
+    constexpr int kSwizzleV = kByRow ? 1 : (G::kChunksPerRowV % 16 == 0 ? 16 : 8);
     auto pieceOf = [](int row, int chunk) { return row * G::kChunksPerRowV + (chunk ^ (row & (kSwizzleV - 1))); };
     uint4 *stage = reinterpret_cast<uint4 *>(&tiles) + w * (R * 16 * G::kChunksPerRowV);
 #pragma unroll
